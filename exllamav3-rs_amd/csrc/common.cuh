@@ -104,6 +104,12 @@ __device__ __forceinline__ float mul_f16_f32(uint32_t pair, float c)
 __device__ __forceinline__ float round_f16(float v) { return (float)to_f16(v); }
 __device__ __forceinline__ float round_bf16(float v) { return bf16lo(pack_bf16(v, 0.0f)); }
 
+// Every tensor is global memory: the accessors say so (address space 1).  Where a pointer's origin is lost to
+// the compiler (a per-lane choice between q, k and v rows as integers) a plain access becomes a flat_load,
+// which counts as an LDS access too, so any later wait for a scalar or LDS read also waits for it.
+template <class T> using gptr = __attribute__((address_space(1))) T*;
+template <class T> using gcptr = const __attribute__((address_space(1))) T*;
+
 // load8: cached load (weights, embedding tables: reused across rows).  load8s: streaming load with
 // the non-temporal hint for operands read exactly once.  store8: every output is written once per
 // call, so all stores carry the non-temporal hint.  (Measured on MI355X: a 1 GiB copy reaches
@@ -117,17 +123,17 @@ template <class T> __device__ __forceinline__ float round_to(float v);
 
 template <> __device__ __forceinline__ TF16::Vec load8<TF16>(const void* base, int64_t e)
 {
-    return { *(const u32x4*)((const uint16_t*)base + e) };
+    return { *(gcptr<u32x4>)((const uint16_t*)base + e) };
 }
 template <> __device__ __forceinline__ TBF16::Vec load8<TBF16>(const void* base, int64_t e)
 {
-    return { *(const u32x4*)((const uint16_t*)base + e) };
+    return { *(gcptr<u32x4>)((const uint16_t*)base + e) };
 }
 template <> __device__ __forceinline__ TF32::Vec load8<TF32>(const void* base, int64_t e)
 {
     // Members are assigned one by one: a braced {p[0], p[1]} would be brace-elided into the
     // elements of the first vector member.
-    const u32x4* p = (const u32x4*)((const float*)base + e);
+    const gcptr<u32x4> p = (gcptr<u32x4>)((const float*)base + e);
     TF32::Vec v;
     v.a = p[0];
     v.b = p[1];
@@ -136,15 +142,15 @@ template <> __device__ __forceinline__ TF32::Vec load8<TF32>(const void* base, i
 
 template <> __device__ __forceinline__ TF16::Vec load8s<TF16>(const void* base, int64_t e)
 {
-    return { __builtin_nontemporal_load((const u32x4*)((const uint16_t*)base + e)) };
+    return { __builtin_nontemporal_load((gcptr<u32x4>)((const uint16_t*)base + e)) };
 }
 template <> __device__ __forceinline__ TBF16::Vec load8s<TBF16>(const void* base, int64_t e)
 {
-    return { __builtin_nontemporal_load((const u32x4*)((const uint16_t*)base + e)) };
+    return { __builtin_nontemporal_load((gcptr<u32x4>)((const uint16_t*)base + e)) };
 }
 template <> __device__ __forceinline__ TF32::Vec load8s<TF32>(const void* base, int64_t e)
 {
-    const u32x4* p = (const u32x4*)((const float*)base + e);
+    const gcptr<u32x4> p = (gcptr<u32x4>)((const float*)base + e);
     TF32::Vec v;
     v.a = __builtin_nontemporal_load(p);
     v.b = __builtin_nontemporal_load(p + 1);
@@ -153,15 +159,15 @@ template <> __device__ __forceinline__ TF32::Vec load8s<TF32>(const void* base, 
 
 template <> __device__ __forceinline__ void store8<TF16>(void* base, int64_t e, const TF16::Vec& v)
 {
-    __builtin_nontemporal_store(v.a, (u32x4*)((uint16_t*)base + e));
+    __builtin_nontemporal_store(v.a, (gptr<u32x4>)((uint16_t*)base + e));
 }
 template <> __device__ __forceinline__ void store8<TBF16>(void* base, int64_t e, const TBF16::Vec& v)
 {
-    __builtin_nontemporal_store(v.a, (u32x4*)((uint16_t*)base + e));
+    __builtin_nontemporal_store(v.a, (gptr<u32x4>)((uint16_t*)base + e));
 }
 template <> __device__ __forceinline__ void store8<TF32>(void* base, int64_t e, const TF32::Vec& v)
 {
-    u32x4* p = (u32x4*)((float*)base + e);
+    const gptr<u32x4> p = (gptr<u32x4>)((float*)base + e);
     __builtin_nontemporal_store(v.a, p);
     __builtin_nontemporal_store(v.b, p + 1);
 }
@@ -171,15 +177,15 @@ template <> __device__ __forceinline__ void store8<TF32>(void* base, int64_t e, 
 template <class T> __device__ __forceinline__ void store8c(void* base, int64_t elem, const typename T::Vec& v);
 template <> __device__ __forceinline__ void store8c<TF16>(void* base, int64_t e, const TF16::Vec& v)
 {
-    *(u32x4*)((uint16_t*)base + e) = v.a;
+    *(gptr<u32x4>)((uint16_t*)base + e) = v.a;
 }
 template <> __device__ __forceinline__ void store8c<TBF16>(void* base, int64_t e, const TBF16::Vec& v)
 {
-    *(u32x4*)((uint16_t*)base + e) = v.a;
+    *(gptr<u32x4>)((uint16_t*)base + e) = v.a;
 }
 template <> __device__ __forceinline__ void store8c<TF32>(void* base, int64_t e, const TF32::Vec& v)
 {
-    u32x4* p = (u32x4*)((float*)base + e);
+    const gptr<u32x4> p = (gptr<u32x4>)((float*)base + e);
     p[0] = v.a;
     p[1] = v.b;
 }
@@ -232,14 +238,14 @@ template <class T> __device__ __forceinline__ void store8_split(void* base, int6
 
 __device__ __forceinline__ u32x4 load16x2_split(const uint16_t* p)
 {
-    const u32x2 lo = __builtin_nontemporal_load((const u32x2*)p);
-    const u32x2 hi = __builtin_nontemporal_load((const u32x2*)(p + kSplitGap));
+    const u32x2 lo = __builtin_nontemporal_load((gcptr<u32x2>)p);
+    const u32x2 hi = __builtin_nontemporal_load((gcptr<u32x2>)(p + kSplitGap));
     return u32x4{ lo.x, lo.y, hi.x, hi.y };
 }
 __device__ __forceinline__ void store16x2_split(uint16_t* p, u32x4 v)
 {
-    __builtin_nontemporal_store(u32x2{ v.x, v.y }, (u32x2*)p);
-    __builtin_nontemporal_store(u32x2{ v.z, v.w }, (u32x2*)(p + kSplitGap));
+    __builtin_nontemporal_store(u32x2{ v.x, v.y }, (gptr<u32x2>)p);
+    __builtin_nontemporal_store(u32x2{ v.z, v.w }, (gptr<u32x2>)(p + kSplitGap));
 }
 template <> __device__ __forceinline__ TF16::Vec load8s_split<TF16>(const void* base, int64_t e)
 {
@@ -253,15 +259,15 @@ template <> __device__ __forceinline__ TF32::Vec load8s_split<TF32>(const void* 
 {
     const float* p = (const float*)base + e;
     TF32::Vec v;
-    v.a = __builtin_nontemporal_load((const u32x4*)p);
-    v.b = __builtin_nontemporal_load((const u32x4*)(p + kSplitGap));
+    v.a = __builtin_nontemporal_load((gcptr<u32x4>)p);
+    v.b = __builtin_nontemporal_load((gcptr<u32x4>)(p + kSplitGap));
     return v;
 }
 // Cached form (hot embedding-table rows).
 template <class T> __device__ __forceinline__ typename T::Vec load8_split(const void* base, int64_t e);
 __device__ __forceinline__ u32x4 load16x2_split_cached(const uint16_t* p)
 {
-    const u32x2 lo = *(const u32x2*)p, hi = *(const u32x2*)(p + kSplitGap);
+    const u32x2 lo = *(gcptr<u32x2>)p, hi = *(gcptr<u32x2>)(p + kSplitGap);
     return u32x4{ lo.x, lo.y, hi.x, hi.y };
 }
 template <> __device__ __forceinline__ TF16::Vec load8_split<TF16>(const void* base, int64_t e)
@@ -276,8 +282,8 @@ template <> __device__ __forceinline__ TF32::Vec load8_split<TF32>(const void* b
 {
     const float* p = (const float*)base + e;
     TF32::Vec v;
-    v.a = *(const u32x4*)p;
-    v.b = *(const u32x4*)(p + kSplitGap);
+    v.a = *(gcptr<u32x4>)p;
+    v.b = *(gcptr<u32x4>)(p + kSplitGap);
     return v;
 }
 
@@ -292,8 +298,8 @@ template <> __device__ __forceinline__ void store8_split<TBF16>(void* base, int6
 template <> __device__ __forceinline__ void store8_split<TF32>(void* base, int64_t e, const TF32::Vec& v)
 {
     float* p = (float*)base + e;
-    __builtin_nontemporal_store(v.a, (u32x4*)p);
-    __builtin_nontemporal_store(v.b, (u32x4*)(p + kSplitGap));
+    __builtin_nontemporal_store(v.a, (gptr<u32x4>)p);
+    __builtin_nontemporal_store(v.b, (gptr<u32x4>)(p + kSplitGap));
 }
 
 template <> __device__ __forceinline__ void unpack8<TF16>(const TF16::Vec& v, float (&f)[8])
@@ -349,15 +355,15 @@ template <> __device__ __forceinline__ float round_to<TBF16>(float v) { return r
 // Scalar element access (generic fallback kernels).
 __device__ __forceinline__ float load1(const void* p, int dt, int64_t i)
 {
-    if (dt == DT_F16) return (float)((const _Float16*)p)[i];
-    if (dt == DT_BF16) return __builtin_bit_cast(float, (uint32_t)((const uint16_t*)p)[i] << 16);
-    return ((const float*)p)[i];
+    if (dt == DT_F16) return (float)((gcptr<_Float16>)p)[i];
+    if (dt == DT_BF16) return __builtin_bit_cast(float, (uint32_t)((gcptr<uint16_t>)p)[i] << 16);
+    return ((gcptr<float>)p)[i];
 }
 __device__ __forceinline__ void store1(void* p, int dt, int64_t i, float v)
 {
-    if (dt == DT_F16) ((_Float16*)p)[i] = to_f16(v);
-    else if (dt == DT_BF16) ((uint16_t*)p)[i] = (uint16_t)(pack_bf16(v, 0.0f) & 0xffffu);
-    else ((float*)p)[i] = v;
+    if (dt == DT_F16) ((gptr<_Float16>)p)[i] = to_f16(v);
+    else if (dt == DT_BF16) ((gptr<uint16_t>)p)[i] = (uint16_t)(pack_bf16(v, 0.0f) & 0xffffu);
+    else ((gptr<float>)p)[i] = v;
 }
 __device__ __forceinline__ float round1(float v, int dt)
 {
@@ -460,45 +466,6 @@ constexpr int DPP_ROW_HALF_MIRROR = 0x141;
 constexpr int DPP_ROW_MIRROR = 0x140;
 constexpr int DPP_ROW_ROR8 = 0x128;
 
-// Sum over aligned groups of W lanes (W = 1, 2, 4, ..., 64); every lane of a group gets the sum.
-// Must be called with the whole wave active.
-template <int W>
-__device__ __forceinline__ float group_sum(float v)
-{
-    if constexpr (W >= 2) v += dpp<DPP_QUAD_XOR1>(v);
-    if constexpr (W >= 4) v += dpp<DPP_QUAD_XOR2>(v);
-    if constexpr (W >= 8) v += dpp<DPP_ROW_HALF_MIRROR>(v);
-    if constexpr (W >= 16) v += dpp<DPP_ROW_MIRROR>(v);
-    if constexpr (W >= 32)
-        v += __builtin_bit_cast(float, __builtin_amdgcn_ds_swizzle(__builtin_bit_cast(int, v), 0x401f)); // xor 16
-    if constexpr (W >= 64)
-        v += __shfl_xor(v, 32);
-    return v;
-}
-
-template <int CTRL>
-__device__ __forceinline__ double dpp64(double v)
-{
-    const uint64_t u = __builtin_bit_cast(uint64_t, v);
-    const int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, CTRL, 0xf, 0xf, false);
-    const int hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), CTRL, 0xf, 0xf, false);
-    return __builtin_bit_cast(double, ((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
-}
-
-// fp64 group sum (as group_sum): used where the statistic must match a double-precision oracle
-// bit-for-bit after rounding to fp32.
-template <int W>
-__device__ __forceinline__ double group_sum64(double v)
-{
-    if constexpr (W >= 2) v += dpp64<DPP_QUAD_XOR1>(v);
-    if constexpr (W >= 4) v += dpp64<DPP_QUAD_XOR2>(v);
-    if constexpr (W >= 8) v += dpp64<DPP_ROW_HALF_MIRROR>(v);
-    if constexpr (W >= 16) v += dpp64<DPP_ROW_MIRROR>(v);
-    if constexpr (W >= 32) v += __shfl_xor(v, 16);
-    if constexpr (W >= 64) v += __shfl_xor(v, 32);
-    return v;
-}
-
 // v(l) + v(l ^ 16) in every lane l: v_permlane16_swap_b32 of v with itself hands both lanes of a pair
 // the pair's two values in the same order (the even row's first), so both get the same bits.  Both
 // lanes of a pair must be active.
@@ -521,6 +488,12 @@ __device__ __forceinline__ double sum_xor16(double v)
 
 // v(l) + v(l ^ 32) in every lane l, the same bits in both (v_permlane32_swap_b32 of v with itself: the
 // lower half's value first).  Both lanes of a pair must be active.
+__device__ __forceinline__ float sum_xor32(float v)
+{
+    const uint32_t u = __builtin_bit_cast(uint32_t, v);
+    const auto p = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+    return __builtin_bit_cast(float, (uint32_t)p[0]) + __builtin_bit_cast(float, (uint32_t)p[1]);
+}
 __device__ __forceinline__ double sum_xor32(double v)
 {
     const uint64_t u = __builtin_bit_cast(uint64_t, v);
@@ -530,6 +503,45 @@ __device__ __forceinline__ double sum_xor32(double v)
     const double a = __builtin_bit_cast(double, ((uint64_t)(uint32_t)ph[0] << 32) | (uint32_t)pl[0]);
     const double b = __builtin_bit_cast(double, ((uint64_t)(uint32_t)ph[1] << 32) | (uint32_t)pl[1]);
     return a + b;
+}
+
+// Sum over aligned groups of W lanes (W = 1, 2, 4, ..., 64); every lane of a group gets the sum.
+// Must be called with the whole wave active.  Lanes 16 and 32 apart meet through the permlane swaps, which
+// stay in the VALU: a ds_bpermute there is an LDS round trip in a chain that nothing else hides when a
+// launch has one row (the same sums in the same order).
+template <int W>
+__device__ __forceinline__ float group_sum(float v)
+{
+    if constexpr (W >= 2) v += dpp<DPP_QUAD_XOR1>(v);
+    if constexpr (W >= 4) v += dpp<DPP_QUAD_XOR2>(v);
+    if constexpr (W >= 8) v += dpp<DPP_ROW_HALF_MIRROR>(v);
+    if constexpr (W >= 16) v += dpp<DPP_ROW_MIRROR>(v);
+    if constexpr (W >= 32) v = sum_xor16(v);
+    if constexpr (W >= 64) v = sum_xor32(v);
+    return v;
+}
+
+template <int CTRL>
+__device__ __forceinline__ double dpp64(double v)
+{
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, CTRL, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), CTRL, 0xf, 0xf, false);
+    return __builtin_bit_cast(double, ((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
+}
+
+// fp64 group sum (as group_sum): used where the statistic must match a double-precision oracle
+// bit-for-bit after rounding to fp32.
+template <int W>
+__device__ __forceinline__ double group_sum64(double v)
+{
+    if constexpr (W >= 2) v += dpp64<DPP_QUAD_XOR1>(v);
+    if constexpr (W >= 4) v += dpp64<DPP_QUAD_XOR2>(v);
+    if constexpr (W >= 8) v += dpp64<DPP_ROW_HALF_MIRROR>(v);
+    if constexpr (W >= 16) v += dpp64<DPP_ROW_MIRROR>(v);
+    if constexpr (W >= 32) v = sum_xor16(v);
+    if constexpr (W >= 64) v = sum_xor32(v);
+    return v;
 }
 
 // Full-wave sum, uniform result: row sums by DPP, then the four rows combined through readlane.
@@ -572,6 +584,17 @@ __device__ __forceinline__ double block_sum64(double v, double* lds16)
     return t;
 }
 
+// Sum of the nw <= 16 wave partials in LDS: lane l of every 16-lane row reads partial l, one read for the
+// wave instead of nw reads in a chain, and the row's DPP butterfly adds them.  Every lane gets the sum.
+template <class T>
+__device__ __forceinline__ T lds_partials_sum(const T* lds16, int nw)
+{
+    const int l = threadIdx.x & 15;
+    const T v = l < nw ? lds16[l] : (T)0;
+    if constexpr (sizeof(T) == 8) return group_sum64<16>(v);
+    else return group_sum<16>(v);
+}
+
 // fp64 workgroup sum with a single barrier, for a workgroup that reduces once: its LDS slots are
 // never written again, so no second barrier is needed before the kernel ends.
 __device__ __forceinline__ double block_sum64_once(double v, double* lds16)
@@ -581,9 +604,7 @@ __device__ __forceinline__ double block_sum64_once(double v, double* lds16)
     if (nw == 1) return v;
     if ((threadIdx.x & 63) == 0) lds16[threadIdx.x >> 6] = v;
     __syncthreads();
-    double t = 0.0;
-    for (int i = 0; i < nw; ++i) t += lds16[i];
-    return t;
+    return lds_partials_sum(lds16, nw);
 }
 
 // Workgroup sum with a single barrier (see block_sum64_once), for an fp64 or fp32 partial.
@@ -595,9 +616,7 @@ __device__ __forceinline__ float block_sum_once(float v, float* lds16)
     if (nw == 1) return v;
     if ((threadIdx.x & 63) == 0) lds16[threadIdx.x >> 6] = v;
     __syncthreads();
-    float t = 0.0f;
-    for (int i = 0; i < nw; ++i) t += lds16[i];
-    return t;
+    return lds_partials_sum(lds16, nw);
 }
 
 // ---------------------------------------------------------------------------------------------

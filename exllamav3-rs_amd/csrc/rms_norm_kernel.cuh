@@ -569,6 +569,15 @@ __device__ __forceinline__ void rms_finish(const RmsArgs& a, int64_t row, int ti
     }
 }
 
+// Has every argument that a row's loads, sums and stores use fetched at the kernel's entry, by one batch of
+// scalar loads.  Left alone, the compiler sinks each argument's load into the branch that uses it, and a
+// launch of one row then waits for two or three round trips to the argument segment before its first HBM load.
+__device__ __forceinline__ void rms_fetch_args(const RmsArgs& a)
+{
+    asm volatile("" : : "s"(a.x), "s"(a.ldx), "s"(a.r), "s"(a.ldr), "s"(a.w), "s"(a.wt), "s"(a.y), "s"(a.ldy),
+                        "s"(a.row0), "s"(a.dim), "s"(a.eps), "s"(a.cb), "s"(a.cs));
+}
+
 // One row per workgroup: its loads, pass 1, one reduction, pass 2.  (A grid-stride loop over rows, with
 // the second barrier it needs before LDS reuse, measured ~1 us slower at [8192, 5120].)
 template <class XT, class YT, class RT, int MAXV, int MODE, int HAD = 0, int WM = W_EARLY, bool SPLIT = false,
@@ -577,6 +586,7 @@ __global__ __launch_bounds__(1024) void k_rms_norm(RmsArgs a)
 {
     static_assert(!SPLIT || (HAD == 0 && (MODE == RMS_PLAIN || MODE == RMS_RES_IN)), "split chunks: plain and residual norms");
     __shared__ ACC red[16];
+    rms_fetch_args(a);
     const int64_t row = a.row0 + blockIdx.x;
     RowRegs<XT, RT, MAXV> L;
     rms_load<XT, RT, MAXV, MODE, SPLIT, HAD>(a, row, threadIdx.x, blockDim.x, WM == W_EARLY, L);
