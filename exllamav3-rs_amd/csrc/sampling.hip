@@ -40,6 +40,7 @@ struct ArgArgs
     int64_t rows;
     uint64_t* ids;
     uint32_t seed;       // Gumbel noise key
+    int64_t slice;       // elements per slice of the sliced kernels (a multiple of 2048)
 };
 
 // Philox4x32-10: ten rounds of two 32 x 32 -> 64-bit products with the published multipliers,
@@ -121,19 +122,6 @@ __device__ __forceinline__ float gumbel1(uint32_t seed, int64_t row, int64_t c)
 }
 
 // Candidate value: the logit, plus its noise for a Gumbel draw.
-template <bool GUMBEL>
-__device__ __forceinline__ void candidates8(float (&f)[8], const ArgArgs& a, int64_t row, int64_t c)
-{
-    #pragma clang fp contract(off)
-    if constexpr (GUMBEL)
-    {
-        float g[8];
-        gumbel8(a.seed, row, c, g);
-        #pragma unroll
-        for (int j = 0; j < 8; ++j) f[j] = f[j] + g[j];
-    }
-}
-
 template <bool GUMBEL>
 __device__ __forceinline__ float candidate1(const char* base, int dt, const ArgArgs& a, int64_t row, int64_t c)
 {
@@ -266,22 +254,194 @@ __global__ __launch_bounds__(256) void k_argmax_convert(uint64_t* ids, int64_t r
     }
 }
 
-// One lane's best candidate over its UNROLL chunks of the slice starting at `start` of `row`.  VEC:
-// 16-byte aligned rows, whole chunks loaded as vectors (a chunk crossing n is read element by
-// element); otherwise every element is read on its own.
+// A whole chunk of 8 logits.  ALIGNED: 16-byte aligned rows; otherwise (an odd vocabulary, a sliced tensor)
+// the same 16-byte accesses at the alignment of one element, which the hardware splits where they cross a
+// line, in place of 8 single reads and, for a draw, 8 Philox blocks instead of 2 (64 x 151935 f32 logits, us,
+// before and after: argmax 24.6 -> 13.6, draw 34.8 -> 15.4).
+typedef u32x4 __attribute__((aligned(2))) u32x4_u2;
+typedef u32x4 __attribute__((aligned(4))) u32x4_u4;
+template <class IT, bool ALIGNED>
+__device__ __forceinline__ typename IT::Vec load_chunk(const void* base, int64_t c)
+{
+    if constexpr (ALIGNED) return load8s<IT>(base, c);
+    else if constexpr (IT::code == DT_F32)
+    {
+        const gcptr<u32x4_u4> p = (gcptr<u32x4_u4>)((const float*)base + c);
+        typename IT::Vec v;
+        v.a = __builtin_nontemporal_load(p);
+        v.b = __builtin_nontemporal_load(p + 1);
+        return v;
+    }
+    else return { __builtin_nontemporal_load((gcptr<u32x4_u2>)((const uint16_t*)base + c)) };
+}
+
+// ---------------------------------------------------------------------------------------------
+// The Gumbel draw's candidates.  The noise is the cost of a draw: its two logs as log_f32 evaluates them are
+// 60 of 80 VALU instructions per element.  Only the winner's noise has to be that exact, so the draw first
+// ranks every candidate with the hardware's log2 (v_log_f32), which needs 5 instructions, and then evaluates
+// log_f32's noise for the candidates that come within a bound of the best rank, one as a rule.
+//
+// b = x - ln2 log2(-log2 u) is the candidate x + g less the constant -ln ln 2.  Over all 2^23 values of u
+// the noise part differs from g by less than kRankErr (tests/test_gpu_gumbel.py walks them), and forming b and
+// x + g rounds each by at most 2^-24 of its size, so with m the largest b, a candidate with
+// b < m - (2 kRankErr + 2^-20 |m|) is below the one that has b = m: |b| <= 2 |m| leaves 3 * 2^-23 |m| for the
+// roundings, and a larger |b| (b far below m) is more than |b| / 2 away.  The best candidate, and any that
+// ties with it, is therefore always evaluated, and the draw is the same index as before.
+// A NaN or infinite m (NaN or +inf logits, or nothing but -inf) takes the exact evaluation of every candidate.
+// The largest difference measured over all u is 1.6e-6.  64 rows of 151936 f32 logits took 22.0 us with
+// every candidate exact, bound by VALU issue, and take 14.7 (three launches, ~13 us of host time from Python); 1024 rows 247 -> 122.5 us (5.1 TB/s).
+constexpr float kRankErr = 1e-5f;
+
+__device__ __forceinline__ float gumbel_rank(float x, uint32_t bits)
+{
+    // u = ((bits >> 9) + 0.5) 2^-23 exactly: 1.mantissa less 1 - 2^-24
+    const float u = __builtin_bit_cast(float, __builtin_amdgcn_alignbit(0x7fu, bits, 9)) - 0x1.fffffep-1f;
+    return __builtin_fmaf(__builtin_amdgcn_logf(-__builtin_amdgcn_logf(u)), -0x1.62e43p-1f, x);
+}
+__device__ __forceinline__ float rank_floor(float m) { return m - __builtin_fmaf(fabsf(m), 0x1p-20f, 2.0f * kRankErr); }
+__device__ __forceinline__ float max_nan(float a, float b) { return __builtin_elementwise_maximum(a, b); }
+__device__ __forceinline__ float wave_max_nan(float v)
+{
+    v = max_nan(v, dpp<DPP_QUAD_XOR1>(v));
+    v = max_nan(v, dpp<DPP_QUAD_XOR2>(v));
+    v = max_nan(v, dpp<DPP_ROW_HALF_MIRROR>(v));
+    v = max_nan(v, dpp<DPP_ROW_MIRROR>(v));
+    const uint32_t u = __builtin_bit_cast(uint32_t, v);
+    const auto p = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    v = max_nan(__builtin_bit_cast(float, (uint32_t)p[0]), __builtin_bit_cast(float, (uint32_t)p[1]));
+    const uint32_t w = __builtin_bit_cast(uint32_t, v);
+    const auto q = __builtin_amdgcn_permlane32_swap(w, w, false, false);
+    return max_nan(__builtin_bit_cast(float, (uint32_t)q[0]), __builtin_bit_cast(float, (uint32_t)q[1]));
+}
+
+// The chunk's 8 logits (-inf past the row), from the loaded vector or, for a chunk that crosses n, one by one.
+template <class IT>
+__device__ __forceinline__ void chunk_logits(const ArgArgs& a, const char* base, const typename IT::Vec& v, int64_t c, float (&x)[8])
+{
+    if (c + 8 <= a.n) unpack8<IT>(v, x);
+    else
+    {
+        #pragma unroll
+        for (int j = 0; j < 8; ++j) x[j] = c + j < a.n ? load1(base, IT::code, c + j) : -INFINITY;
+    }
+}
+
+__device__ __forceinline__ void chunk_ranks(const float (&x)[8], uint32_t seed, int64_t row, int64_t c, uint32_t (&w)[8],
+                                            float (&k)[8])
+{
+    #pragma unroll
+    for (int h = 0; h < 2; ++h)
+    {
+        uint32_t q[4];
+        philox4x32_10((uint32_t)(c >> 2) + h, (uint32_t)row, (uint32_t)((uint64_t)row >> 32), 0u, seed, 0u, q);
+        #pragma unroll
+        for (int j = 0; j < 4; ++j)
+        {
+            w[4 * h + j] = q[j];
+            k[4 * h + j] = gumbel_rank(x[4 * h + j], q[j]);
+        }
+    }
+}
+
+// The exact candidates of the chunk at c whose rank reaches `floor`, in index order.
+template <class IT, bool VEC>
+__device__ __forceinline__ void take_chunk(const ArgArgs& a, const char* base, int64_t row, int64_t c, float floor, LaneBest& lb)
+{
+    #pragma clang fp contract(off)
+    typename IT::Vec v{};
+    if (c + 8 <= a.n) v = load_chunk<IT, VEC>(base, c);
+    float x[8], k[8];
+    uint32_t w[8], left = 0;
+    chunk_logits<IT>(a, base, v, c, x);
+    chunk_ranks(x, a.seed, row, c, w, k);
+    #pragma unroll
+    for (int j = 0; j < 8; ++j) left |= c + j < a.n && k[j] >= floor ? 1u << j : 0u;
+    while (left)
+    {
+        const int j = __builtin_ctz(left);
+        left &= left - 1;
+        float xj = x[0];
+        uint32_t wj = w[0];
+        #pragma unroll
+        for (int i = 1; i < 8; ++i)
+        {
+            xj = j == i ? x[i] : xj;
+            wj = j == i ? w[i] : wj;
+        }
+        lb.consider(xj + gumbel_of_bits(wj), c + j);
+    }
+}
+
+// One lane's best candidate of the draw over elements [start, end) of `row`, end at most n, by a workgroup of
+// THREADS lanes (every lane must get here; wmax: one LDS slot per wave).  A lane walks its chunks start + 8 tid,
+// + 8 THREADS, ... keeping the largest chunk rank, that chunk, and the largest rank of its other chunks; the
+// workgroup's largest rank then decides which chunk is looked at again.  (As a rolled loop with the next
+// chunk's load issued ahead: unrolled four times it holds 140 VGPRs, 3 waves per SIMD.)
+template <class IT, bool VEC, int THREADS>
+__device__ __forceinline__ uint64_t gumbel_lane_key(const ArgArgs& a, int64_t row, int64_t start, int64_t end, int tid,
+                                                    float* wmax)
+{
+    const char* base = a.x + row * a.ld;
+    constexpr int STEP = THREADS * 8;
+    float top = -INFINITY, other = -INFINITY;
+    int64_t at = start + tid * 8;
+    typename IT::Vec v{}, vn{};
+    if (at + 8 <= a.n && at < end) v = load_chunk<IT, VEC>(base, at);
+    #pragma unroll 1
+    for (int64_t c = at; c < end; c += STEP)
+    {
+        const int64_t cn = c + STEP;
+        if (cn + 8 <= a.n && cn < end) vn = load_chunk<IT, VEC>(base, cn);
+        float x[8], k[8];
+        uint32_t w[8];
+        chunk_logits<IT>(a, base, v, c, x);
+        chunk_ranks(x, a.seed, row, c, w, k);
+        const float m = max_nan(max_nan(max_nan(k[0], k[1]), max_nan(k[2], k[3])), max_nan(max_nan(k[4], k[5]), max_nan(k[6], k[7])));
+        other = fmaxf(other, fminf(top, m));
+        at = m > top ? c : at;
+        top = max_nan(top, m);
+        v = vn;
+    }
+    const float mw = wave_max_nan(top);
+    if ((tid & 63) == 0) wmax[tid >> 6] = mw;
+    __syncthreads();
+    float m = wmax[0];
+    #pragma unroll
+    for (int i = 1; i < THREADS / 64; ++i) m = max_nan(m, wmax[i]);
+    const bool finite = fabsf(m) < INFINITY;
+    const float floor = finite ? rank_floor(m) : 0.0f;
+    LaneBest lb;
+    if (!finite || other >= floor)      // NaN or infinities about, or two chunks of a lane this close: all of them
+    {
+        for (int64_t c = start + tid * 8; c < end; c += STEP)
+            for (int j = 0; j < 8 && c + j < end; ++j) lb.consider(candidate1<true>(base, IT::code, a, row, c + j), c + j);
+    }
+    else if (top >= floor)
+        take_chunk<IT, VEC>(a, base, row, at, floor, lb);
+    return lb.key();
+}
+
+// One lane's best candidate over its UNROLL chunks of the slice starting at `start` of `row`.  A chunk crossing
+// n is read element by element.  GUMBEL: the workgroup's largest rank (wmax: one LDS slot per wave) decides
+// which candidates are evaluated; every lane of the workgroup must get here.
 template <class IT, bool VEC, int UNROLL, bool GUMBEL>
-__device__ __forceinline__ uint64_t slice_lane_key(const ArgArgs& a, int64_t row, int64_t start, int tid)
+__device__ __forceinline__ uint64_t slice_lane_key(const ArgArgs& a, int64_t row, int64_t start, int tid, float* wmax)
 {
     const char* base = a.x + row * a.ld;
     LaneBest lb;
+    if constexpr (GUMBEL)
+    {
+        const int64_t end = start + a.slice;
+        return gumbel_lane_key<IT, VEC, 256>(a, row, start, end < a.n ? end : a.n, tid, wmax);
+    }
     typename IT::Vec v[UNROLL];
     #pragma unroll
     for (int u = 0; u < UNROLL; ++u)
     {
         const int64_t c = start + u * 2048 + tid * 8;
-        if (VEC && c + 8 <= a.n) v[u] = load8s<IT>(base, c);
+        if (c + 8 <= a.n) v[u] = load_chunk<IT, VEC>(base, c);
     }
-    if constexpr (VEC && IT::code == DT_F16 && !GUMBEL)
+    if constexpr (IT::code == DT_F16)
     {
         // whole chunks by LaneBestF16 (a chunk is whole only when every earlier one of the lane is)
         LaneBestF16 hb;
@@ -301,19 +461,17 @@ __device__ __forceinline__ uint64_t slice_lane_key(const ArgArgs& a, int64_t row
     for (int u = 0; u < UNROLL; ++u)
     {
         const int64_t c = start + u * 2048 + tid * 8;
-        if (VEC && c + 8 <= a.n)
+        if (c + 8 <= a.n)
         {
-            if constexpr (IT::code == DT_F16 && !GUMBEL) continue;   // taken above
+            if constexpr (IT::code == DT_F16) continue;   // taken above
             float f[8];
             unpack8<IT>(v[u], f);
-            candidates8<GUMBEL>(f, a, row, c);
             #pragma unroll
             for (int j = 0; j < 8; ++j) lb.consider(f[j], c + j);
         }
         else
         {
-            for (int j = 0; j < 8 && c + j < a.n; ++j)
-                lb.consider(candidate1<GUMBEL>(base, IT::code, a, row, c + j), c + j);
+            for (int j = 0; j < 8 && c + j < a.n; ++j) lb.consider(load1(base, IT::code, c + j), c + j);
         }
     }
     return lb.key();
@@ -326,11 +484,12 @@ template <class IT, bool VEC, int UNROLL, bool GUMBEL>
 __global__ __launch_bounds__(256) void k_argmax(ArgArgs a)
 {
     __shared__ uint64_t part[4];
+    __shared__ float wmax[4];
     const int tid = threadIdx.x;
-    const int64_t start = (int64_t)blockIdx.x * UNROLL * 2048;
+    const int64_t start = (int64_t)blockIdx.x * a.slice;
     for (int64_t row = blockIdx.y; row < a.rows; row += gridDim.y)
     {
-        uint64_t best = wave_max_u64(slice_lane_key<IT, VEC, UNROLL, GUMBEL>(a, row, start, tid));
+        uint64_t best = wave_max_u64(slice_lane_key<IT, VEC, UNROLL, GUMBEL>(a, row, start, tid, wmax));
         if ((tid & 63) == 0) part[tid >> 6] = best;
         __syncthreads();
         if (tid == 0)
@@ -356,12 +515,13 @@ template <class IT, bool VEC, int UNROLL, bool GUMBEL>
 __global__ __launch_bounds__(256) void k_argmax_ws(ArgArgs a, uint32_t* count, uint64_t* slot)
 {
     __shared__ uint64_t wpart[4];
+    __shared__ float wmax[4];
     const int tid = threadIdx.x;
     const uint32_t slices = gridDim.x;
-    const int64_t start = (int64_t)blockIdx.x * UNROLL * 2048;
+    const int64_t start = (int64_t)blockIdx.x * a.slice;
     for (int64_t row = blockIdx.y; row < a.rows; row += gridDim.y)
     {
-        uint64_t best = wave_max_u64(slice_lane_key<IT, VEC, UNROLL, GUMBEL>(a, row, start, tid));
+        uint64_t best = wave_max_u64(slice_lane_key<IT, VEC, UNROLL, GUMBEL>(a, row, start, tid, wmax));
         if ((tid & 63) == 0) wpart[tid >> 6] = best;
         __syncthreads();
         if (tid == 0)
@@ -391,12 +551,18 @@ __global__ __launch_bounds__(THREADS) void k_argmax_rows(ArgArgs a)
     constexpr int WAVES = THREADS / 64;
     constexpr int STEP = THREADS * 8;          // elements per chunk round
     __shared__ uint64_t part[WAVES];
+    __shared__ float wmax[WAVES];
     const int tid = threadIdx.x;
     for (int64_t row = blockIdx.x; row < a.rows; row += gridDim.x)
     {
         const char* base = a.x + row * a.ld;
         LaneBest lb;
-        if constexpr (VEC && IT::code == DT_F16 && !GUMBEL)
+        [[maybe_unused]] uint64_t lane_key = 0;
+        if constexpr (GUMBEL)
+        {
+            lane_key = gumbel_lane_key<IT, VEC, THREADS>(a, row, 0, a.n, tid, wmax);
+        }
+        else if constexpr (IT::code == DT_F16)
         {
             // whole chunks by LaneBestF16, then the elements of a partial last chunk (after every whole
             // one) by the lane that holds it
@@ -408,7 +574,7 @@ __global__ __launch_bounds__(THREADS) void k_argmax_rows(ArgArgs a)
                 for (int u = 0; u < 4; ++u)
                 {
                     const int64_t c = s0 + u * STEP + tid * 8;
-                    if (c < nw) v[u] = load8s<TF16>(base, c).a;
+                    if (c < nw) v[u] = load_chunk<TF16, VEC>(base, c).a;
                 }
                 #pragma unroll
                 for (int u = 0; u < 4; ++u)
@@ -434,28 +600,26 @@ __global__ __launch_bounds__(THREADS) void k_argmax_rows(ArgArgs a)
             for (int u = 0; u < 4; ++u)
             {
                 const int64_t c = s0 + u * STEP + tid * 8;
-                if (VEC && c + 8 <= a.n) v[u] = load8s<IT>(base, c);
+                if (c + 8 <= a.n) v[u] = load_chunk<IT, VEC>(base, c);
             }
             #pragma unroll
             for (int u = 0; u < 4; ++u)
             {
                 const int64_t c = s0 + u * STEP + tid * 8;
-                if (VEC && c + 8 <= a.n)
+                if (c + 8 <= a.n)
                 {
                     float f[8];
                     unpack8<IT>(v[u], f);
-                    candidates8<GUMBEL>(f, a, row, c);
                     #pragma unroll
                     for (int j = 0; j < 8; ++j) lb.consider(f[j], c + j);
                 }
                 else
                 {
-                    for (int j = 0; j < 8 && c + j < a.n; ++j)
-                        lb.consider(candidate1<GUMBEL>(base, IT::code, a, row, c + j), c + j);
+                    for (int j = 0; j < 8 && c + j < a.n; ++j) lb.consider(load1(base, IT::code, c + j), c + j);
                 }
             }
         }
-        uint64_t best = wave_max_u64(lb.key());
+        uint64_t best = wave_max_u64(GUMBEL ? lane_key : lb.key());
         if ((tid & 63) == 0) part[tid >> 6] = best;
         __syncthreads();
         if (tid == 0)
@@ -583,14 +747,15 @@ int sample_entry(const char* op, const void* logits, int dtype, int64_t rows, in
     if (!logits || !ids) return set_error(EXL3R_EINVAL, "%s: logits and ids must be non-null", op);
     const int64_t n = (max_logit <= 0 || max_logit > vocab) ? vocab : max_logit;
     const int es = dtype_bytes(dtype);
-    ArgArgs a{ (const char*)logits, (rows > 1 ? ld : vocab) * es, n, rows, (uint64_t*)ids, seed };
+    ArgArgs a{ (const char*)logits, (rows > 1 ? ld : vocab) * es, n, rows, (uint64_t*)ids, seed, 0 };
     hipStream_t s = (hipStream_t)stream;
     const bool vec = aligned16(logits) && a.ld % 16 == 0;
     // Measured on MI355X over f16 [rows, 151936] logits (us; sliced / a workgroup per row with 512 /
     // 1024 lanes): argmax 64 rows 11.2 / 25.0 / 16.4, 128 rows 16.8 / 25.7 / 17.0, 192 rows 21.8 /
-    // 26.3 / 17.4, 512 rows - / 32.0 / 33.5 (256 lanes 57.0), 1024 rows - / 62.3 / 64.5; the Gumbel
-    // draw, compute-bound, keeps the sliced kernel longer: 256 rows 58.9 / 74.6 / 64.3, 512 rows
-    // 147.6 (256 lanes) / 125.9 / 125.6, 1024 rows - / 225.3 / 246.3.
+    // 26.3 / 17.4, 512 rows - / 32.0 / 33.5 (256 lanes 57.0), 1024 rows - / 62.3 / 64.5.  The Gumbel draw keeps
+    // the sliced kernel longer (f16: 383 rows sliced 44.6, 400 rows by rows 55.3, 1024 rows 96.2; f32 48.8 /
+    // 54.4 / 122.5, when every candidate was evaluated exactly 121.5 / 227.7 and 119.8 / 247.1 at 400 / 1024),
+    // up to the rows that the workspace holds.
     const Tuning& tu = tuning();
     const int64_t rows_min = tu.sample_rows_min > 0 ? tu.sample_rows_min : GUMBEL ? 384 : 128;
     if (rows >= rows_min)
@@ -618,8 +783,14 @@ int sample_entry(const char* op, const void* logits, int dtype, int64_t rows, in
         });
         return launch_status(op);
     }
-    const int unroll = slice_unroll(rows);
-    const int64_t slice = (int64_t)unroll * 2048;
+    const int unroll = GUMBEL ? 1 : slice_unroll(rows);   // (chunks in flight per lane; the draw's loop has its own)
+    int64_t slice = (int64_t)unroll * 2048;
+    // The draw's slices are longer: each costs its workgroup a reduction, the winner's evaluation and an atomic
+    // (us for slices of 2048 / 4096 / 6144 / 8192 / 10240 / 12288 / 16384 f32 logits, 151936 a row, with the
+    // ~13 us of three launches from Python as the floor: 16 rows 16.4 / 13 / 13 / 13 / 13 / 13 / 13, 64 rows
+    // 28.1 / 19.1 / 16.8 / 15.7 / 15.2 / 16.1 / 15.8, 256 rows 62.6 / 42.8 / 37.4 / 37.6 / 35.8 / 36.5 / 38.3).
+    if (GUMBEL && rows >= 16) slice = 5 * 2048;
+    a.slice = slice;
     const dim3 grid((unsigned)((n + slice - 1) / slice), (unsigned)rows);
     if (ws.scratch)
     {
@@ -639,10 +810,10 @@ int sample_entry(const char* op, const void* logits, int dtype, int64_t rows, in
         uint64_t* part = (uint64_t*)((char*)ws.base + kCountBytes);
         with_float_type(dtype, [&](auto T) {
             using Ty = decltype(T);
-            if (unroll == 4)
+            if (!GUMBEL && unroll == 4)
             {
-                if (vec) launch(k_argmax_ws<Ty, true, 4, GUMBEL>, grid, 256, 0, s, a, count, part);
-                else launch(k_argmax_ws<Ty, false, 4, GUMBEL>, grid, 256, 0, s, a, count, part);
+                if (vec) launch(k_argmax_ws<Ty, true, GUMBEL ? 1 : 4, GUMBEL>, grid, 256, 0, s, a, count, part);
+                else launch(k_argmax_ws<Ty, false, GUMBEL ? 1 : 4, GUMBEL>, grid, 256, 0, s, a, count, part);
             }
             else
             {
@@ -656,10 +827,10 @@ int sample_entry(const char* op, const void* logits, int dtype, int64_t rows, in
     launch(k_argmax_clear, small, 256, 0, s, a.ids, rows);
     with_float_type(dtype, [&](auto T) {
         using Ty = decltype(T);
-        if (unroll == 4)
+        if (!GUMBEL && unroll == 4)
         {
-            if (vec) launch(k_argmax<Ty, true, 4, GUMBEL>, grid, 256, 0, s, a);
-            else launch(k_argmax<Ty, false, 4, GUMBEL>, grid, 256, 0, s, a);
+            if (vec) launch(k_argmax<Ty, true, GUMBEL ? 1 : 4, GUMBEL>, grid, 256, 0, s, a);
+            else launch(k_argmax<Ty, false, GUMBEL ? 1 : 4, GUMBEL>, grid, 256, 0, s, a);
         }
         else
         {

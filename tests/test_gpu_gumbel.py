@@ -130,3 +130,26 @@ def test_zero_rows_and_cols():
     y = torch.empty((4, 0), device="cuda")
     ffi.gumbel_noise(y, y, 1)
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("rows,vocab,width", [(1, 151936, 0.0), (16, 40961, 1e-5), (64, 151936, 1e-4), (400, 20011, 3e-6)])
+def test_sample_near_ties(rows, vocab, width):
+    """Logits that undo the noise to within `width` (0: to the rounding of the sum), so that almost every
+    candidate comes within the bound that decides which ones the draw evaluates exactly, on both kernels and on
+    rows of every alignment.  The draw is the oracle's, which evaluates all of them."""
+    noise = torch.empty((rows, vocab), dtype=torch.float32, device="cuda")
+    ffi.gumbel_noise(torch.zeros_like(noise), noise, 91)
+    g = torch.Generator(device="cuda").manual_seed(92)
+    x = 1.5 - noise - width * torch.rand((rows, vocab), generator=g, device="cuda")
+    run_sample(x, F32, 91)
+    run_sample((x + 1e4)[:, 1:], F32, 93)
+
+
+@pytest.mark.parametrize("rows", [2, 400])
+def test_sample_masks_of_the_lowest_value(rows):
+    """Rows of the type's lowest value, whose rank bound leaves the float range, alone and with live logits."""
+    for dt, low in ((F16, -65504.0), (BF16, -3.3895313892515355e38), (F32, -3.4028234663852886e38)):
+        x = np.full((rows, 12295), low, np.float32)
+        x[1::2, 5000:5010] = np.linspace(-2, 2, 10)
+        x[1::2, 12294] = 1.0
+        run_sample(to_dev(orc.to_bits(x, dt), dt), dt, 94)
