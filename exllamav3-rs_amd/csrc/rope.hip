@@ -16,7 +16,8 @@
 // Layout: a head of head_dim elements is held by LPH = head_dim / 8 lanes, 8 elements (16 bytes) per
 // lane, so a wave holds 64 / LPH heads (4 heads of 128).  The head sum is a DPP butterfly inside the
 // LPH-lane group; NeoX partners live R/16 lanes apart in the same group and are exchanged by DPP
-// (a rotation by 8 lanes for R = 128) or ds_bpermute, GPT-J partners sit in the same lane.  Two
+// (a rotation by 8 lanes for R = 128) or ds_bpermute, GPT-J partners sit in the same lane.  Heads of 64, 128
+// and 256 take k_rope_nx, which holds 16 elements per lane with every rotary pair in one lane; the others two
 // kernels: k_rope_tok (prefill NeoX) gives each wave whole tokens -- the token's sin/cos evaluated
 // once, one per lane, and its heads walked in software-pipelined batches; k_rope (decode, GPT-J)
 // flattens (token, head) items over workgroups that share the sin/cos of the tokens they span
@@ -693,11 +694,12 @@ __global__ __launch_bounds__(256) void k_rope_tok(RopeArgs a)
 // (W waves in the grid), so the waves in flight sweep the rows in order; the next item's loads (and
 // its {cos, sin} table row) are issued before the current item is computed.  Evaluated rotary pairs:
 // one sin / cos per lane into the wave's LDS row, once per token within a run.
-template <class IO, int NORM, int SRC, int P>
+template <class IO, int NORM, int SRC, int P, int L>
 struct NxItem
 {
     typename IO::Vec lo[P], hi[P];
     float4 cs[4];                // SRC_CS: the lane's 8 {cos, sin} pairs as loaded
+    float ang[L == 16 ? 2 : 1];  // SRC_ANGLE: the token's angles l64 (and 64 + l64), 0 outside the table
     int64_t tok;
     int64_t crow;                // APPEND: the token's cache row (cache_row), -1: none or not needed
     int slice;
@@ -823,22 +825,47 @@ __device__ __forceinline__ double nx_head_sum(double v)
         return group_sum64<8>(v);
 }
 
-template <class IO, int MODE, int NORM, int SRC, bool QOUT, int P, bool APPEND = false, int HADR = HADR_NONE>
+// L lanes per head of 16 L elements (4: 64, 8: 128, 16: 256), 64 / L heads per pass.  PART (NeoX only): a
+// rotary width R of 16 m elements, R / 2 = 8 m apart.  Lane j < m of a head holds the chunks j and j + m,
+// whose elements pair up; lane j >= m holds the chunks m + j and L + j past the rotary width, which are
+// normed and pass through.  Every pair stays in one lane, as in the full-width layout, which is m = L.
+template <class IO, int MODE, int NORM, int SRC, bool QOUT, int P, bool APPEND = false, int HADR = HADR_NONE, int L = 8,
+          bool PART = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kNxMinWaves<APPEND, HADR, SRC>)))
-void k_rope_nx(RopeArgs a, int nslice, int run)
+void k_rope_nx(RopeArgs a, int nslice, int run, int early)
 {
     static_assert(!(APPEND || HADR) || (P == 1 && !QOUT), "paged / rotating items are single passes");
     static_assert(!HADR || IO::code == DT_F16, "output rotation: f16 heads");
-    extern __shared__ float2 cs[];            // [4 waves][64] (SRC_FREQ)
+    static_assert(!PART || (MODE == EXL3R_ROPE_NEOX && !HADR), "partial widths: NeoX");
+    static_assert(PART || L == 8, "the full-width layout is heads of 128");
+    constexpr int HD = 16 * L;                // head_dim
+    constexpr int HPP = 64 / L;               // heads per pass
+    constexpr int ROW = L == 16 ? 128 : 64;   // {cos, sin} slots per wave: R / 2 at most
+    constexpr bool EVAL = SRC != SRC_CS;      // rotary pairs evaluated in the kernel
+    extern __shared__ float2 cs[];            // [4 waves][ROW] (EVAL)
     // Norm weights with the constant bias folded in, q then k: h(w + h(cb)) (NORM_HALF) or w + cb (NORM_F32).
-    __shared__ __align__(16) float wsh[256];
-    static_assert(SRC == SRC_FREQ || SRC == SRC_CS, "angle tables take the flattened kernel");
+    __shared__ __align__(16) float wsh[2 * HD];
+    // The arguments of the setup and the first item, fetched at entry by one batch of scalar loads (as
+    // rms_fetch_args: each would otherwise be a round trip of its own in front of the first load).
+    asm volatile("" : : "s"(a.q), "s"(a.k), "s"(a.q_ts), "s"(a.q_hs), "s"(a.k_ts), "s"(a.k_hs), "s"(a.hq), "s"(a.hk),
+                        "s"(a.R), "s"(a.tokens), "s"(a.seq_len), "s"(a.position), "s"(a.positions), "s"(a.position_ids),
+                        "s"(a.qw), "s"(a.kw), "s"(a.ns_m), "s"(a.ns_l), "s"(nslice), "s"(run), "s"(early));
+    if constexpr (SRC == SRC_FREQ) asm volatile("" : : "s"(a.inv_freq));
+    if constexpr (APPEND)
+        asm volatile("" : : "s"(a.v), "s"(a.v_ts), "s"(a.v_hs), "s"(a.hv), "s"(a.page_log2), "s"(a.pages),
+                            "s"(a.max_blocks), "s"(a.block_table), "s"(a.cache_seqlens));
     const int l64 = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int64_t W = (int64_t)gridDim.x * 4;
     const int64_t items = a.tokens * nslice;
-    const int grp = nx_head_of_lane<HADR>(l64);   // head of a pass held by this lane
-    const int e0 = nx_e0_of_lane<HADR>(l64);      // the lane's chunks: [e0, e0 + 8) and [e0 + 64, e0 + 72)
+    const int R = a.R, R2 = a.R >> 1;
+    const int grp = PART ? l64 / L : nx_head_of_lane<HADR>(l64);   // head of a pass held by this lane
+    // The lane's chunks: [e0, e0 + 8) and [e0 + gap, e0 + gap + 8); tr: its first rotary pair.
+    const int pj = l64 % L, pm = R >> 4;
+    const bool rot = !PART || pj < pm;            // the lane holds rotary pairs
+    const int e0 = PART ? 8 * (rot ? pj : pm + pj) : nx_e0_of_lane<HADR>(l64);
+    const int gap = PART ? 8 * (rot ? pm : L - pm) : 64;
+    const int tr = PART && !rot ? 0 : e0;
     constexpr bool MF = HADR == HADR_MFMA;
     // had128_mfma's placement: the lane's chunk of each span (index bits 3-6 = lane bits 0, 1, 4, 5) and
     // its head inside the span (lane bits 2-3).
@@ -861,18 +888,25 @@ void k_rope_nx(RopeArgs a, int nslice, int run)
     char* const qout = (char*)a.oq;
     char* const kout = (char*)a.ok;
     const int64_t oq_ts = QOUT ? a.oq_ts : q_ts, oq_hs = QOUT ? a.oq_hs : q_hs;
-    const int R = a.R, R2 = a.R >> 1;
-    using Item = NxItem<IO, NORM, SRC, P>;
-    int64_t evaluated = -1;                   // SRC_FREQ: the token whose pairs the wave's LDS row holds
+    using Item = NxItem<IO, NORM, SRC, P, L>;
+    int64_t evaluated = -1;                   // EVAL: the token whose pairs the wave's LDS row holds
     // SRC_FREQ: the lane's rotary frequency inv_freq[l64], staged through LDS with the norm weights, so
     // that the item loop's only vector loads are the items' own (a wait for an evaluation's read of
     // inv_freq would also wait for the next item's loads).
-    __shared__ float fsh[SRC == SRC_FREQ ? 64 : 1];
-    float freq = 0.0f;
+    __shared__ float fsh[SRC == SRC_FREQ ? ROW : 1];
+    float freq[L == 16 ? 2 : 1] = {};
 
-    // Loads of one item: the lane's two chunks of head (slice * P + p) * 8 + grp for each of the P passes,
-    // and its rotary pairs (SRC_CS) or the token's position (SRC_FREQ).
-    auto issue = [&](Item& t, int64_t item) __attribute__((always_inline)) {
+    // ONE (few items, see the end of the kernel): the lane's own norm weights and post-scales of its head.
+    struct
+    {
+        u32x4 wl, wh;            // NORM_HALF: h(w + h(cb))
+        float fl[8], fh[8];      // NORM_F32: w + cb
+        u32x4 pl, ph;            // HADR post-scales
+    } one;
+
+    // Loads of one item: the lane's two chunks of head (slice * P + p) * HPP + grp for each of the P passes,
+    // and its rotary pairs (SRC_CS), its angles (SRC_ANGLE) or the token's position (SRC_FREQ).
+    auto issue_data = [&](Item& t, int64_t item) __attribute__((always_inline)) {
         t.tok = (int64_t)udiv_magic((uint64_t)item, a.ns_m, a.ns_l);   // item / nslice
         t.slice = (int)(item - t.tok * nslice);
         // The row of head h of token tok.
@@ -904,13 +938,13 @@ void k_rope_nx(RopeArgs a, int nslice, int run)
             }
             else
             {
-                const char* base = head_base(min((t.slice * P + p) * 8 + grp, H - 1));
+                const char* base = head_base(min((t.slice * P + p) * HPP + grp, H - 1));
                 t.lo[p] = load8s<IO>(base, e0);
-                t.hi[p] = load8s<IO>(base, e0 + 64);
+                t.hi[p] = load8s<IO>(base, e0 + gap);
             }
         }
-        // The cache row, once per item that holds k or v heads (wave-uniform).
-        if constexpr (APPEND) t.crow = (t.slice + 1) * 8 > hq ? cache_row_u(a, t.tok) : -1;
+    };
+    auto issue_pairs = [&](Item& t) __attribute__((always_inline)) {
         if constexpr (SRC == SRC_CS)
         {
             // NeoX: pairs e0 .. e0 + 7; GPT-J: pairs e0/2 .. e0/2 + 3 (lo chunk) and 32 + e0/2 .. (hi chunk)
@@ -918,7 +952,7 @@ void k_rope_nx(RopeArgs a, int nslice, int run)
             if constexpr (MODE == EXL3R_ROPE_NEOX)
             {
                 #pragma unroll
-                for (int i = 0; i < 4; ++i) t.cs[i] = ((const float4*)(row + e0))[i];
+                for (int i = 0; i < 4; ++i) t.cs[i] = ((const float4*)(row + tr))[i];
             }
             else
             {
@@ -930,53 +964,40 @@ void k_rope_nx(RopeArgs a, int nslice, int run)
                 }
             }
         }
+        else if constexpr (SRC == SRC_ANGLE)
+        {
+            // The token's row of the angle table, one angle per lane, fetched with the item's data; a
+            // position outside the table sets *err and rotates by 0.
+            const int pos = token_position_u(a, t.tok);
+            const bool in = pos >= 0 && pos < a.table_rows;
+            if (!in && a.err) atomicOr(a.err, 1);
+            const float* row = a.table + token_seq_u(a, t.tok) * a.table_bstride + (int64_t)(in ? pos : 0) * R2;
+            #pragma unroll
+            for (int i = 0; i < (int)(sizeof(t.ang) / 4); ++i)
+                t.ang[i] = in ? row[min(l64 + 64 * i, R2 - 1)] : 0.0f;
+        }
         else
             t.pos = token_position_u(a, t.tok);
     };
+    auto issue = [&](Item& t, int64_t item) __attribute__((always_inline)) {
+        issue_data(t, item);
+        // The cache row, once per item that holds k or v heads (wave-uniform).
+        if constexpr (APPEND) t.crow = (t.slice + 1) * HPP > hq ? cache_row_u(a, t.tok) : -1;
+        issue_pairs(t);
+    };
+    const int64_t item0 = ((int64_t)blockIdx.x * 4 + wave) * run;
 
-    if constexpr (NORM != NORM_NONE)
-    {
-        const int i = threadIdx.x, e = i & 127;
-        const void* w = i < 128 ? a.qw : a.kw;
-        if constexpr (NORM == NORM_HALF)
-        {
-            _Float16* wh = (_Float16*)wsh;
-            wh[i] = w ? ((const _Float16*)w)[e] + to_f16(a.cb) : (_Float16)0.0f;
-        }
-        else
-            wsh[i] = w ? load1(w, a.wt, e) + a.cb : 0.0f;
-    }
-    if constexpr (SRC == SRC_FREQ)
-        if (threadIdx.x < 64) fsh[threadIdx.x] = (int)threadIdx.x < R2 ? a.inv_freq[threadIdx.x] : 0.0f;
     // HADR: the post-scales of all H heads (item-space order, 128 halfs each; zeros for a projection
     // without one, never read) into LDS after the {cos, sin} rows, 16 bytes per thread and step, so that
     // an item's read of them is an LDS read, whose wait does not also wait for the next item's loads.
     // (Indexed as an LDS array: a generic pointer into it trips an instruction-selection error in hipcc,
     // ROCm 7.2, for the comparisons of the flat address.)
     extern __shared__ u32x4 dyn16[];          // the dynamic LDS in 16-byte units
-    constexpr int kPost16 = SRC == SRC_FREQ ? 4 * 64 * 8 / 16 : 0;
-    if constexpr (HADR != HADR_NONE)
-    {
-        for (int i = threadIdx.x; i < H * 16; i += 256)
-        {
-            const int h = i >> 4;
-            const bool iq = h < hq, iv = APPEND && h >= hq + hk;
-            const int hi = h - (iq ? 0 : hq) - (iv ? hk : 0);
-            const void* p = pick_qkv(iq, iv, qpost, kpost, vpost);
-            u32x4 v = {};
-            if (p) v = *(const u32x4*)((const _Float16*)p + (int64_t)hi * 128 + (i & 15) * 8);
-            dyn16[kPost16 + i] = v;
-        }
-    }
-    if constexpr (NORM != NORM_NONE || SRC == SRC_FREQ || HADR != HADR_NONE)
-    {
-        __syncthreads();
-        if constexpr (SRC == SRC_FREQ) freq = fsh[l64];
-    }
-
+    constexpr int kPost16 = EVAL ? 4 * ROW * 8 / 16 : 0;
     // Head norm, rotation and stores of one pass (lo / hi: the lane's chunks of head h < H).
     auto pass = [&](int64_t tok, int h, typename IO::Vec& lo, typename IO::Vec& hi, const float (&c)[8],
-                    const float (&s)[8], int64_t crow) __attribute__((always_inline)) {
+                    const float (&s)[8], auto&& cache_row_of, auto ONE) __attribute__((always_inline)) {
+        constexpr bool one_item = decltype(ONE)::value;
         const bool isq = h < hq;
         const bool isv = APPEND && h >= hq + hk;
         const int hidx = h - (isq ? 0 : hq) - (isv ? hk : 0);
@@ -989,7 +1010,12 @@ void k_rope_nx(RopeArgs a, int nslice, int run)
             const bool hp = post != nullptr;
             u32x4 pl = {}, ph = {};
             auto load_post = [&]() __attribute__((always_inline)) {
-                if (hp)
+                if constexpr (one_item)
+                {
+                    pl = one.pl;
+                    ph = one.ph;
+                }
+                else if (hp)
                 {
                     pl = dyn16[kPost16 + h * 16 + (e0 >> 3)];
                     ph = dyn16[kPost16 + h * 16 + (e0 >> 3) + 8];
@@ -1040,6 +1066,7 @@ void k_rope_nx(RopeArgs a, int nslice, int run)
             unpack8<IO>(hi, fh);
             // fp64 sum of squares (as rope_head: exact for 16-bit data, one rounding to fp32)
             float mean;
+#ifdef EXL3R_TUNING
             if (a.ss32)
             {
                 float s32 = 0.0f;
@@ -1047,24 +1074,35 @@ void k_rope_nx(RopeArgs a, int nslice, int run)
                 for (int j = 0; j < 8; ++j) s32 = fmaf(fl[j], fl[j], s32);
                 #pragma unroll
                 for (int j = 0; j < 8; ++j) s32 = fmaf(fh[j], fh[j], s32);
-                mean = nx_head_sum<HADR>(s32) * a.inv_hd;
+                mean = (PART ? group_sum<L>(s32) : nx_head_sum<HADR>(s32)) * a.inv_hd;
             }
             else
+#endif
             {
                 double ss = 0.0;
                 #pragma unroll
                 for (int j = 0; j < 8; ++j) ss = fma((double)fl[j], (double)fl[j], ss);
                 #pragma unroll
                 for (int j = 0; j < 8; ++j) ss = fma((double)fh[j], (double)fh[j], ss);
-                ss = nx_head_sum<HADR>(ss);
-                mean = (float)ss * a.inv_hd;     // head_dim 128: an exact multiply
+                if constexpr (PART) ss = group_sum64<L>(ss);
+                else ss = nx_head_sum<HADR>(ss);
+                mean = (float)ss * a.inv_hd;     // head_dim 64, 128, 256: an exact multiply
             }
             const float rmf = 1.0f / sqrtf(mean + a.eps);
-            const int wo = (isq ? 0 : 128) + e0;
+            const int wo = (isq ? 0 : HD) + e0;
             if constexpr (NORM == NORM_HALF)
             {
-                const u32x4 wl = *(const u32x4*)((const _Float16*)wsh + wo);
-                const u32x4 wh = *(const u32x4*)((const _Float16*)wsh + wo + 64);
+                u32x4 wl, wh;
+                if constexpr (one_item)
+                {
+                    wl = one.wl;
+                    wh = one.wh;
+                }
+                else
+                {
+                    wl = *(const u32x4*)((const _Float16*)wsh + wo);
+                    wh = *(const u32x4*)((const _Float16*)wsh + wo + gap);
+                }
                 #pragma unroll
                 for (int i = 0; i < 4; ++i)
                 {
@@ -1083,8 +1121,8 @@ void k_rope_nx(RopeArgs a, int nslice, int run)
                 #pragma unroll
                 for (int j = 0; j < 8; ++j)
                 {
-                    fl[j] = opaque((fl[j] * rmf) * wsh[wo + j]);
-                    fh[j] = opaque((fh[j] * rmf) * wsh[wo + 64 + j]);
+                    fl[j] = opaque((fl[j] * rmf) * (one_item ? one.fl[j] : wsh[wo + j]));
+                    fh[j] = opaque((fh[j] * rmf) * (one_item ? one.fh[j] : wsh[wo + gap + j]));
                 }
                 lo = pack8<IO>(fl);
                 hi = pack8<IO>(fh);
@@ -1093,6 +1131,7 @@ void k_rope_nx(RopeArgs a, int nslice, int run)
         {
             // r1 = fl(fl(v1 c) - fl(v2 s)), r2 = fl(fl(v2 c) + fl(v1 s)), each rounded once to io.
             #pragma clang fp contract(off)
+            [[maybe_unused]] const typename IO::Vec plo = lo, phi = hi;   // PART: the chunks that pass through
             if constexpr (MODE == EXL3R_ROPE_NEOX && IO::code == DT_F16)
             {
                 // The products straight from the packed f16 pairs (no unpacking; the same roundings).
@@ -1163,6 +1202,15 @@ void k_rope_nx(RopeArgs a, int nslice, int run)
                 lo = pack8<IO>(fl);
                 hi = pack8<IO>(fh);
             }
+            if constexpr (PART)
+            {
+                #pragma unroll
+                for (int i = 0; i < 4; ++i)
+                {
+                    lo.a[i] = rot ? lo.a[i] : plo.a[i];
+                    hi.a[i] = rot ? hi.a[i] : phi.a[i];
+                }
+            }
         }
         }
         if (isq || (!isv && (!APPEND || kout)))
@@ -1180,22 +1228,23 @@ void k_rope_nx(RopeArgs a, int nslice, int run)
                 oo = (int32_t)((int64_t)hidx * k_hs) + e0;
             }
             store8<IO>(ob, oo, lo);
-            store8<IO>(ob, oo + 64, hi);
+            store8<IO>(ob, oo + gap, hi);
         }
         if constexpr (APPEND)
         {
+            const int64_t crow = cache_row_of();
             if (!isq && crow >= 0)
             {
                 char* cb = isv ? vcache : kcache;
-                const int64_t co = crow + (int64_t)hidx * 128 + e0;
+                const int64_t co = crow + (int64_t)hidx * HD + e0;
                 store8<IO>(cb, co, lo);
-                store8<IO>(cb, co + 64, hi);
+                store8<IO>(cb, co + gap, hi);
             }
         }
     };
 
-    auto compute = [&](Item& t) __attribute__((always_inline)) {
-        float c[8], s[8];
+    // The lane's cos / sin of an item: read, or evaluated into the wave's LDS row once per token within a run.
+    auto pairs = [&](Item& t, float (&c)[8], float (&s)[8]) __attribute__((always_inline)) {
         if constexpr (SRC == SRC_CS)
         {
             #pragma unroll
@@ -1209,11 +1258,21 @@ void k_rope_nx(RopeArgs a, int nslice, int run)
         }
         else
         {
-            float2* row = cs + wave * 64;
+            float2* row = cs + wave * ROW;
             if (t.tok != evaluated)           // wave-uniform: once per token within a run
             {
                 wave_lds_sync();
-                if (MODE == EXL3R_ROPE_NEOX || l64 < R2) row[l64] = rope_cs_of_angle(__fmul_rn(freq, (float)t.pos), a.attn);
+                #pragma unroll
+                for (int i = 0; i < ROW / 64; ++i)
+                {
+                    if (!(PART || MODE != EXL3R_ROPE_NEOX) || l64 + 64 * i < R2)
+                    {
+                        float ang;
+                        if constexpr (SRC == SRC_ANGLE) ang = t.ang[i];
+                        else ang = __fmul_rn(freq[i], (float)t.pos);
+                        row[l64 + 64 * i] = rope_cs_of_angle(ang, a.attn);
+                    }
+                }
                 wave_lds_sync();
                 evaluated = t.tok;
             }
@@ -1221,19 +1280,157 @@ void k_rope_nx(RopeArgs a, int nslice, int run)
             for (int j = 0; j < 8; ++j)
             {
                 // NeoX: pair e0 + j; GPT-J: pair e0/2 + j (lo chunk, j < 4) or 32 + e0/2 + j - 4 (hi chunk)
-                const int tp = MODE == EXL3R_ROPE_NEOX ? e0 + j : j < 4 ? e0 / 2 + j : 32 + e0 / 2 + (j - 4);
+                const int tp = MODE == EXL3R_ROPE_NEOX ? tr + j : j < 4 ? e0 / 2 + j : 32 + e0 / 2 + (j - 4);
                 const float2 x = MODE == EXL3R_ROPE_NEOX || tp < R2 ? row[tp] : make_float2(0.0f, 0.0f);   // NeoX: R2 = 64
                 c[j] = x.x;
                 s[j] = x.y;
             }
         }
-        #pragma unroll
-        for (int p = 0; p < P; ++p)
-            if (p == 0 || (t.slice * P + p) * 8 < H)   // wave-uniform: a pass past the last head is skipped whole
-                pass(t.tok, min((t.slice * P + p) * 8 + grp, H - 1), t.lo[p], t.hi[p], c, s, APPEND ? t.crow : -1);
     };
 
-    int64_t item = ((int64_t)blockIdx.x * 4 + wave) * run;
+    auto compute = [&](Item& t) __attribute__((always_inline)) {
+        float c[8], s[8];
+        pairs(t, c, s);
+        #pragma unroll
+        for (int p = 0; p < P; ++p)
+            if (p == 0 || (t.slice * P + p) * HPP < H)   // wave-uniform: a pass past the last head is skipped whole
+                pass(t.tok, min((t.slice * P + p) * HPP + grp, H - 1), t.lo[p], t.hi[p], c, s,
+                     [&] { return APPEND ? t.crow : -1; }, std::false_type{});
+    };
+
+    if constexpr (P == 1)
+    {
+    // Few items (a decode batch, a short prefill): every wave has one at most.  Such a launch is one chain of
+    // latencies, so everything an item needs is loaded at once, the weights and post-scales straight into the
+    // lanes that use them: no LDS setup, no barrier, and the rotary pairs are evaluated while the loads are in
+    // flight.  The page of the cache row is a vector load that only the stores wait for.  RoPE and paged append
+    // of 64 / 8 heads, HIP graph, us before and after: 1 token 3.49 -> 2.86, 64 sequences 3.81 -> 3.55.  (Sending
+    // the item's loads ahead of the LDS setup and then entering the loop below gained nothing: the loop's
+    // registers are others, and moving a loaded value waits for it.)
+    if (early)
+    {
+        if (item0 >= items) return;
+        Item A;
+        issue_data(A, item0);
+        const int h = min(A.slice * HPP + grp, H - 1);
+        if constexpr (NORM != NORM_NONE)
+        {
+            const void* w = h < hq ? a.qw : a.kw;
+            if constexpr (NORM == NORM_HALF)
+            {
+                one.wl = load8<TF16>(w, e0).a;
+                one.wh = load8<TF16>(w, e0 + gap).a;
+            }
+            else
+            {
+                load8_dyn(w, a.wt, e0, one.fl);
+                load8_dyn(w, a.wt, e0 + gap, one.fh);
+            }
+        }
+        if constexpr (HADR != HADR_NONE)
+        {
+            const bool iq = h < hq, iv = APPEND && h >= hq + hk;
+            const void* post = pick_qkv(iq, iv, qpost, kpost, vpost);
+            if (post)
+            {
+                const int64_t c = (int64_t)(h - (iq ? 0 : hq) - (iv ? hk : 0)) * 128 + e0;
+                one.pl = load8<TF16>(post, c).a;
+                one.ph = load8<TF16>(post, c + 64).a;
+            }
+        }
+        if constexpr (SRC == SRC_FREQ)
+        {
+            #pragma unroll
+            for (int i = 0; i < (int)(sizeof(freq) / 4); ++i) freq[i] = ((gcptr<float>)a.inv_freq)[min(l64 + 64 * i, R2 - 1)];
+        }
+        int page = -1, slot = 0;
+        const bool kv = APPEND && (A.slice + 1) * HPP > hq;      // wave-uniform
+        if (kv)
+        {
+            const int64_t b = token_seq_u(a, A.tok);
+            const int64_t pos = (int64_t)scalar_i32(a.cache_seqlens, b) + (A.tok - b * a.seq_len);
+            const int64_t lb = pos >> a.page_log2;
+            slot = (int)(pos & (((int64_t)1 << a.page_log2) - 1));
+            int zero;
+            asm volatile("v_mov_b32 %0, 0" : "=v"(zero));
+            if (pos >= 0 && lb < a.max_blocks) page = ((gcptr<int32_t>)a.block_table)[b * a.max_blocks + lb + zero];
+        }
+        issue_pairs(A);
+        float c[8], s[8];
+        pairs(A, c, s);
+        if constexpr (NORM == NORM_HALF)
+        {
+            const _Float16 cbh = to_f16(a.cb);
+            const f16x2 cb2 = { cbh, cbh };
+            #pragma unroll
+            for (int i = 0; i < 4; ++i)
+            {
+                one.wl[i] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, (uint32_t)one.wl[i]) + cb2);
+                one.wh[i] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, (uint32_t)one.wh[i]) + cb2);
+            }
+        }
+        else if constexpr (NORM == NORM_F32)
+        {
+            #pragma unroll
+            for (int j = 0; j < 8; ++j)
+            {
+                one.fl[j] = one.fl[j] + a.cb;
+                one.fh[j] = one.fh[j] + a.cb;
+            }
+        }
+        auto crow = [&]() __attribute__((always_inline)) -> int64_t {
+            if (!kv) return -1;
+            if (page < 0 || page >= a.pages)
+            {
+                if (a.err) atomicOr(a.err, 1);
+                return -1;
+            }
+            return (((int64_t)page << a.page_log2) + slot) * hk * HD;
+        };
+        #pragma unroll
+        for (int p = 0; p < P; ++p)
+            if (p == 0) pass(A.tok, h, A.lo[p], A.hi[p], c, s, crow, std::true_type{});
+        return;
+    }
+
+    }
+
+    if constexpr (NORM != NORM_NONE)
+    {
+        for (int i = threadIdx.x; i < 2 * HD; i += 256)
+        {
+            const int e = i & (HD - 1);
+            const void* w = i < HD ? a.qw : a.kw;
+            if constexpr (NORM == NORM_HALF) ((_Float16*)wsh)[i] = w ? ((const _Float16*)w)[e] + to_f16(a.cb) : (_Float16)0.0f;
+            else wsh[i] = w ? load1(w, a.wt, e) + a.cb : 0.0f;
+        }
+    }
+    if constexpr (SRC == SRC_FREQ)
+        if (threadIdx.x < ROW) fsh[threadIdx.x] = (int)threadIdx.x < R2 ? a.inv_freq[threadIdx.x] : 0.0f;
+    if constexpr (HADR != HADR_NONE)
+    {
+        for (int i = threadIdx.x; i < H * 16; i += 256)
+        {
+            const int h = i >> 4;
+            const bool iq = h < hq, iv = APPEND && h >= hq + hk;
+            const int hi = h - (iq ? 0 : hq) - (iv ? hk : 0);
+            const void* p = pick_qkv(iq, iv, qpost, kpost, vpost);
+            u32x4 v = {};
+            if (p) v = *(gcptr<u32x4>)((const _Float16*)p + (int64_t)hi * 128 + (i & 15) * 8);
+            dyn16[kPost16 + i] = v;
+        }
+    }
+    if constexpr (NORM != NORM_NONE || SRC == SRC_FREQ || HADR != HADR_NONE)
+    {
+        __syncthreads();
+        if constexpr (SRC == SRC_FREQ)
+        {
+            #pragma unroll
+            for (int i = 0; i < (int)(sizeof(freq) / 4); ++i) freq[i] = fsh[l64 + 64 * i];
+        }
+    }
+
+    int64_t item = item0;
     if (item >= items) return;
     int j = 0;                                // item's place in its run
     auto next = [&](int64_t it) __attribute__((always_inline)) -> int64_t {
@@ -1268,9 +1465,9 @@ void k_rope_nx(RopeArgs a, int nslice, int run)
     }
 }
 
-// The k_rope_nx launch: head_dim 128 at prefill sizes (NeoX with rotary_dim 128, GPT-J with rotary_dim a
-// multiple of 4), from inv_freq or a 16-byte aligned {cos, sin} table (no angle table), plain, with the
-// paged append, and / or with the output rotations (16-byte aligned post-scales).  The grid walks the
+// The k_rope_nx launch: head_dim 128 (NeoX with rotary_dim 128, GPT-J with rotary_dim a multiple of 4), from
+// inv_freq, a table of angles or a 16-byte aligned {cos, sin} table, plain, with the paged append, and / or with
+// the output rotations (16-byte aligned post-scales; no angle table with either).  The grid walks the
 // items with the workgroups resident at once.
 // had: the launch carries the output rotations (exl3r_rope_had, exl3r_rope_paged_kv_had).
 static bool rope_nx_ok(const RopeArgs& a, int rope_mode, bool had = false)
@@ -1278,8 +1475,9 @@ static bool rope_nx_ok(const RopeArgs& a, int rope_mode, bool had = false)
     const Tuning& tu = tuning();
     auto a16 = [](const void* p) { return p == nullptr || aligned16(p); };
     // GPT-J: rotary_dim % 4 == 0 keeps each 16-byte table read (two pairs) inside the token's row.
-    if (tu.rope_nx < 0 || a.hd != 128 || (rope_mode == EXL3R_ROPE_NEOX ? a.R != 128 : a.R % 4 != 0) || a.table)
+    if (tu.rope_nx < 0 || a.hd != 128 || (rope_mode == EXL3R_ROPE_NEOX ? a.R != 128 : a.R % 4 != 0))
         return false;
+    if (had && a.table) return false;
     if (tu.rope_tok != 0 && tu.rope_nx == 0) return false;   // a test forcing one of the other kernels
     if (a.kc && a.hv != a.hk) return false;
     // the output rotations' post-scales of all heads in LDS: up to 192 heads (48 KB)
@@ -1293,25 +1491,26 @@ static bool rope_nx_ok(const RopeArgs& a, int rope_mode, bool had = false)
     return true;
 }
 
-template <class IO, int MODE, int NORM, int SRC, bool QOUT, int P, bool APPEND = false, int HADR = HADR_NONE>
+template <class IO, int MODE, int NORM, int SRC, bool QOUT, int P, bool APPEND = false, int HADR = HADR_NONE, int L = 8,
+          bool PART = false>
 static void launch_rope_nx_p(const RopeArgs& a, hipStream_t s)
 {
+    constexpr int HPP = 64 / L;
+    constexpr size_t kRows = SRC != SRC_CS ? 4 * (L == 16 ? 128 : 64) * sizeof(float2) : 0;   // {cos, sin} rows
     const int H = a.hq + a.hk + (APPEND ? a.hv : 0);
-    const int nslice = ((H + 7) / 8 + P - 1) / P;
+    const int nslice = ((H + HPP - 1) / HPP + P - 1) / P;
     const int64_t items = a.tokens * nslice;
     // The output rotations' post-scales sit in LDS (H * 256 bytes; rope_nx_ok bounds H).  Up to 96 heads
     // five workgroups of 20 resident waves per CU take at most 130 KB of its 160 KB with the {cos, sin}
     // rows; more heads can lower the occupancy, which is then asked for at the launch.
-    const size_t cs_lds = SRC == SRC_FREQ ? 4 * 64 * sizeof(float2) : 0;
-    const size_t lds = cs_lds + (HADR != HADR_NONE ? (size_t)H * 256 : 0);
-    constexpr size_t kLdsCommon = SRC == SRC_FREQ ? 4 * 64 * sizeof(float2) + (HADR != HADR_NONE ? 24 << 10 : 0)
-                                                  : (HADR != HADR_NONE ? 24 << 10 : 0);
+    const size_t lds = kRows + (HADR != HADR_NONE ? (size_t)H * 256 : 0);
+    constexpr size_t kLdsCommon = kRows + (HADR != HADR_NONE ? 24 << 10 : 0);
     // Grid: the workgroups resident at once (per CU, from the occupancy of this instance), each wave
     // walking its items i, i + W, ...
     auto occupancy = [](size_t bytes) {
         int nb = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_rope_nx<IO, MODE, NORM, SRC, QOUT, P, APPEND, HADR>, 256,
-                                                         bytes) != hipSuccess || nb < 1)
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_rope_nx<IO, MODE, NORM, SRC, QOUT, P, APPEND, HADR, L, PART>,
+                                                         256, bytes) != hipSuccess || nb < 1)
             nb = 4;
         return nb;
     };
@@ -1319,6 +1518,7 @@ static void launch_rope_nx_p(const RopeArgs& a, hipStream_t s)
     const int resident = lds <= kLdsCommon ? resident_common : occupancy(lds);
     const int wpc = tuning().rope_wgs_per_cu;
     int64_t blocks = (int64_t)(wpc > 0 ? wpc : resident) * device_cus();
+    const bool few = items <= blocks * 4;      // a wave per item at most
     // Items a wave takes in a row, its token's angles evaluated once within them, where every wave gets
     // whole runs (prefill sizes).  MI355X, same process, us at runs of 1 / 2 / 3: C4 NeoX 33.2 / 32.1 /
     // 33.3; q / k rotations + RoPE at C4 46.8 / 45.5 / 42.7; q / k / v rotations + RoPE + paged append at
@@ -1328,7 +1528,9 @@ static void launch_rope_nx_p(const RopeArgs& a, hipStream_t s)
     // 42.5 / 38.8 / 39.7 / 38.5 / 39.6, from the table 38.2 / 36.5 / 38.3 / 35.8 / 41.3 (the wave-per-token
     // kernel: 41.7 / 38.8).  The q | g split (rope_qg, Qwen3.5 4096 tokens) at runs of 1 / 2 / 4: 35.4 /
     // 34.7 / 34.5.
-    constexpr int kRun = HADR ? 3 : APPEND ? 4 : SRC == SRC_FREQ && P == 1 ? 2 : 1;
+    // PART heads run best at 1 (us at 1 / 2: q | g split of 16 / 2 heads of 256, 4639 tokens, f16 18.7 / 19.2,
+    // paged append of 32 / 8 heads of 64 13.4 / 14.1).
+    constexpr int kRun = PART ? 1 : HADR ? 3 : APPEND ? 4 : SRC != SRC_CS && P == 1 ? 2 : 1;
     const int tr = tuning().rope_nx_run;
     const int run = tr > 0 ? tr : items >= (int64_t)kRun * blocks * 4 ? kRun : 1;
     const int64_t runs = (items + run - 1) / run;
@@ -1341,7 +1543,52 @@ static void launch_rope_nx_p(const RopeArgs& a, hipStream_t s)
     if (blocks > kMaxGridX) blocks = kMaxGridX;
     RopeArgs b = a;
     udiv_magic_init((uint64_t)nslice, b.ns_m, b.ns_l);
-    launch(k_rope_nx<IO, MODE, NORM, SRC, QOUT, P, APPEND, HADR>, (unsigned)blocks, 256, lds, s, b, nslice, run);
+    const int early = P == 1 && few && run == 1;
+    launch(k_rope_nx<IO, MODE, NORM, SRC, QOUT, P, APPEND, HADR, L, PART>, (unsigned)blocks, 256, lds, s, b, nslice, run,
+           early);
+}
+
+// Heads of 64 and 256, and partial rotary widths of 128 (NeoX): the same kernel with its PART layout (the
+// vector kernels' conditions hold: R % 16 == 0, 16-byte aligned heads).  MI355X, HIP graph, us, against the
+// wave-per-token kernel (flattened below 1024 tokens and for angle tables): q | g split, 16 / 2 heads of 256 with
+// 64 rotary, 4639 tokens bf16 19.6 / 20.9, f16 18.7 / 24.5, 300 tokens 4.1 / 4.5; 32 / 8 heads of 64 with the paged
+// append, 4096 tokens 13.4 / 17.4, 64 sequences of one token of 16 / 8 3.1 / 3.7; angle tables, 16 / 16 heads of 64,
+// 4096 tokens 9.0 / 13.2, 32 / 8 heads of 128 at full width 16.5 / 26.2.  A half-width rotation of 128 touches
+// half lines per access, and plain prefills of it stay with the wave-per-token kernel (f16 19.9 / 19.3 at 4096
+// tokens of 32 / 8 heads; at 500 tokens 4.3 / 5.1).
+static bool rope_tok_launch(const RopeArgs& a);
+static bool rope_nx_part_ok(const RopeArgs& a, int rope_mode)
+{
+    const bool plain = !a.cst && !a.table && !a.kc && a.oq_ts == a.q_ts && a.oq_hs == a.q_hs;
+    if (a.hd == 128 && plain && rope_tok_launch(a)) return false;
+    const Tuning& tu = tuning();
+    if (tu.rope_nx < 0 || rope_mode != EXL3R_ROPE_NEOX || (a.hd != 64 && a.hd != 128 && a.hd != 256)) return false;
+    if (tu.rope_tok != 0 && tu.rope_nx == 0) return false;   // a test forcing one of the other kernels
+    if (a.kc && a.hv != a.hk) return false;
+    if (a.tokens >= ((int64_t)1 << 31)) return false;
+    return !a.cst || ((uintptr_t)a.cst & 15) == 0;
+}
+
+template <class IO, int NORM>
+static void launch_rope_nx_part(const RopeArgs& a, hipStream_t s)
+{
+    const bool qout = a.oq_ts != a.q_ts || a.oq_hs != a.q_hs;
+    constexpr int NEOX = EXL3R_ROPE_NEOX;
+    auto go = [&](auto LL) {
+        constexpr int L = decltype(LL)::value;
+        if (a.kc)
+        {
+            if (a.cst) launch_rope_nx_p<IO, NEOX, NORM, SRC_CS, false, 1, true, HADR_NONE, L, true>(a, s);
+            else launch_rope_nx_p<IO, NEOX, NORM, SRC_FREQ, false, 1, true, HADR_NONE, L, true>(a, s);
+        }
+        else if (a.cst) launch_rope_nx_p<IO, NEOX, NORM, SRC_CS, false, 1, false, HADR_NONE, L, true>(a, s);
+        else if (a.table) launch_rope_nx_p<IO, NEOX, NORM, SRC_ANGLE, false, 1, false, HADR_NONE, L, true>(a, s);
+        else if (qout) launch_rope_nx_p<IO, NEOX, NORM, SRC_FREQ, true, 1, false, HADR_NONE, L, true>(a, s);
+        else launch_rope_nx_p<IO, NEOX, NORM, SRC_FREQ, false, 1, false, HADR_NONE, L, true>(a, s);
+    };
+    if (a.hd == 64) go(std::integral_constant<int, 4>{});
+    else if (a.hd == 128) go(std::integral_constant<int, 8>{});
+    else go(std::integral_constant<int, 16>{});
 }
 
 // Passes per item: one for NeoX, two for GPT-J (its token's sin / cos or table row shared by two passes).
@@ -1351,7 +1598,7 @@ static void launch_rope_nx_p(const RopeArgs& a, hipStream_t s)
 template <class IO, int MODE, int NORM, int SRC, bool QOUT>
 static void launch_rope_nx(const RopeArgs& a, hipStream_t s)
 {
-    if constexpr (!QOUT)
+    if constexpr (!QOUT && SRC != SRC_ANGLE)   // (no angle table with a paged append)
     {
         if (a.kc)
         {
@@ -1533,8 +1780,6 @@ static void launch_rope_tok(RopeArgs a, hipStream_t s)
     else go(std::integral_constant<int, 3>{});
 }
 
-static bool rope_tok_launch(const RopeArgs& a);
-
 // Prefill-sized NeoX launches (a wave per token still gives every CU several waves) take the
 // wave-per-token kernel.  GPT-J (C4 at rotary 64: 35.2 us flattened vs 37.5 us per token) and
 // decode-sized launches take the flattened kernel: items per lane enough workgroups to fill 256 CUs
@@ -1547,9 +1792,14 @@ static void launch_rope_vec(const RopeArgs& a, int lph, hipStream_t s)
     {
         const bool qout = a.oq_ts != a.q_ts || a.oq_hs != a.q_hs;
         if (a.cst) launch_rope_nx<IO, MODE, NORM, SRC_CS, false>(a, s);
+        else if (a.table) launch_rope_nx<IO, MODE, NORM, SRC_ANGLE, false>(a, s);
         else if (qout) launch_rope_nx<IO, MODE, NORM, SRC_FREQ, true>(a, s);
         else launch_rope_nx<IO, MODE, NORM, SRC_FREQ, false>(a, s);
         return;
+    }
+    if constexpr (MODE == EXL3R_ROPE_NEOX)
+    {
+        if (rope_nx_part_ok(a, MODE)) return launch_rope_nx_part<IO, NORM>(a, s);
     }
     if (a.cst)
     {
