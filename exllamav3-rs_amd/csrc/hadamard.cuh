@@ -403,12 +403,11 @@ __device__ __forceinline__ void mfma_wait_all(MfmaOut (&m)[N])
 // col[n] (mfma_chunk placement), their MFMAs issued together: each transform, one rounding to f16, then
 // the half post-scale (post[n] null: none).
 template <int N>
-__device__ __forceinline__ void output_rotations_mfma(const HadMfma& H, TF16::Vec* v, const void* const* post,
+__device__ __forceinline__ void output_rotations_mfma(HadMfmaWords H, TF16::Vec (&v)[N], const void* const* post,
                                                       const int64_t* col, int lane)
 {
     MfmaOut m[N];
-    #pragma unroll
-    for (int n = 0; n < N; ++n) m[n] = had128_mfma_issue(H, v[n]);
+    had128_mfma_issue_w(H, v, m);
     mfma_wait_all(m);
     #pragma unroll
     for (int n = 0; n < N; ++n)

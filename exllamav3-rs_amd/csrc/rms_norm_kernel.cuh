@@ -70,20 +70,17 @@ constexpr int HAD_OUT = 1;   // rotated f16 outputs, one per projection
 constexpr int HAD_IN = 2;    // x rotated on load
 constexpr int HAD_MFMA = 4;  // the transforms on the matrix cores (had128_mfma)
 
-// The matrix-core transforms need chunk mfma_chunk(l) of a wave's 64-chunk span in lane l, while the
-// row's loads and stores keep chunk l in lane l (with the permuted placement the norm kernels' f32
-// residual and three outputs fetched 1.15x and wrote 1.20x their bytes, against 1.01x and 1.00x with
-// the lane-ordered one: a line's halves come from different rows of a store).  A chunk moves between
-// the two placements through the lane crossbar (ds_bpermute, no LDS storage; the permutation is its own
-// inverse).  Thread counts are multiples of 64, so a wave's chunks c = tid + k * nt are one span of 4
-// blocks for every k.
-__device__ __forceinline__ TF16::Vec mfma_permute(const TF16::Vec& v, int lane)
+// The chunk of a row that a thread owns first (its others follow nt chunks apart).  Matrix-core kernels own
+// chunk mfma_chunk(l) of a wave's 64-chunk span in lane l, the transforms' placement, for every load and store
+// of the row: an access of the wave covers the same span either way, in 64-byte (16-bit) or 128-byte (f32)
+// quads.  (Loading rows in lane order and moving them there and back through the lane crossbar, four ds_bpermute
+// per chunk and direction, cost 0.5 us of 78.5.)  Thread counts are multiples of 64, so a wave's chunks are one
+// span of 4 blocks for every k.
+template <int HAD>
+__device__ __forceinline__ int first_chunk(int tid)
 {
-    const int src = mfma_chunk(lane) << 2;
-    TF16::Vec o;
-    #pragma unroll
-    for (int q = 0; q < 4; ++q) o.a[q] = (uint32_t)__builtin_amdgcn_ds_bpermute(src, (int)v.a[q]);
-    return o;
+    if constexpr ((HAD & HAD_MFMA) != 0) return (tid & ~63) | mfma_chunk(tid & 63);
+    else return tid;
 }
 
 // When a row's weight chunks are fetched (a launch-shape choice: the results are the same bits).
@@ -156,20 +153,29 @@ __device__ __forceinline__ void unpack_w8(u32x4 pre, const void* w, int wt, int6
 }
 
 // Registers of one row between its loads and its arithmetic.
-template <class XT, class RT, int MAXV>
+// pv (matrix-core Hadamard kernels): the consumers' pre-scales of the lane's chunks.  They are loaded with
+// the row, before any store: loads and stores retire through one in-order counter (vmcnt), so a load issued
+// after a store is not waited for without that store's completion in HBM, several microseconds in a busy
+// memory system.  With the pre-scales read where they are used, four such waits made a row's life 15 us and the
+// norm -> three rotations 78.5 us at [4096, 5120] (f16 x, f32 r, rotated input); it takes 69.0, 4.87 TB/s, of
+// 58-62 us for the same streams without arithmetic.
+template <class XT, class RT, int MAXV, int NPRE = 0>
 struct RowRegs
 {
     typename XT::Vec xv[MAXV];
     typename RT::Vec rv[MAXV];
     u32x4 wv[MAXV];
+    u32x4 pv[MAXV][NPRE > 0 ? NPRE : 1];
     bool valid;
 };
+// Pre-scales held per chunk by a kernel (with two chunks per lane they cost 28 VGPRs, 3 of 8 waves per SIMD).
+template <int HAD, int MAXV> constexpr int kRowPre = (HAD & HAD_MFMA) != 0 && MAXV == 1 ? 4 : 0;
 
 // Issues every HBM load of one row -- x (and r) in chunks c = tid, tid + nt, ... (at most MAXV per
 // lane), plus the weight chunks when load_w -- before any arithmetic.
 template <class XT, class RT, int MAXV, int MODE, bool SPLIT = false, int HAD = 0>
 __device__ __forceinline__ void rms_load(const RmsArgs& a, int64_t row, int tid, int nt, bool load_w,
-                                         RowRegs<XT, RT, MAXV>& L)
+                                         RowRegs<XT, RT, MAXV, kRowPre<HAD, MAXV>>& L)
 {
     const int nc = a.dim >> 3;
     const char* xrow;
@@ -191,7 +197,7 @@ __device__ __forceinline__ void rms_load(const RmsArgs& a, int64_t row, int tid,
     #pragma unroll
     for (int k = 0; k < MAXV; ++k)
     {
-        const int c = tid + k * nt;
+        const int c = first_chunk<HAD>(tid) + k * nt;
         const int64_t e = chunk_elem<SPLIT>(c);
         if constexpr ((HAD & HAD_MFMA) != 0)
         {
@@ -221,6 +227,18 @@ __device__ __forceinline__ void rms_load(const RmsArgs& a, int64_t row, int tid,
                 else L.rv[k] = load8s<RT>(rrow, e);
             }
             if (load_w && a.w) L.wv[k] = prefetch_w8<SPLIT>(a.w, a.wt, weight_row<MODE>(a, row) + e);
+        }
+    }
+    if constexpr (kRowPre<HAD, MAXV> > 0)
+    {
+        const int64_t pre = pre_row(a, row);
+        #pragma unroll
+        for (int k = 0; k < MAXV; ++k)
+        {
+            const int c = first_chunk<HAD>(tid) + k * nt;
+            #pragma unroll
+            for (int i = 0; i < kRowPre<HAD, MAXV>; ++i)
+                if (i < a.nh && a.hpre[i]) L.pv[k][i] = load8<TF16>(a.hpre[i], pre + (c < nc ? c * 8 : 0)).a;
         }
     }
 }
@@ -404,21 +422,19 @@ __device__ __forceinline__ void rms_chunk2(const RmsArgs& a, int64_t row, char* 
 // float (one fp32 FMA chain per lane in chunk order, then the wave butterfly and the cross-wave sum in
 // a fixed order: the reference's own precision, norm.cu:101-108, 140-151).
 template <class XT, class YT, class RT, int MAXV, int MODE, int HAD, int WM, bool SPLIT = false, class ACC = double>
-__device__ __forceinline__ void rms_finish(const RmsArgs& a, int64_t row, int tid, int nt, RowRegs<XT, RT, MAXV>& L,
-                                           ACC* red)
+__device__ __forceinline__ void rms_finish(const RmsArgs& a, int64_t row, int tid, int nt,
+                                           RowRegs<XT, RT, MAXV, kRowPre<HAD, MAXV>>& L, ACC* red)
 {
     const int nc = a.dim >> 3;
     char* rrow = (char*)a.r + row * a.ldr * RT::bytes;
     char* yrow = (char*)a.y + row * a.ldy * YT::bytes;
     constexpr bool MF = (HAD & HAD_MFMA) != 0;
-    const int c0 = tid;
+    const int c0 = first_chunk<HAD>(tid);
     const int lane = tid & 63;
-    // chunk held in the matrix-core placement: chunk k of the lane's wave, mfma_chunk(lane) within it
-    [[maybe_unused]] const int cp0 = (tid & ~63) | mfma_chunk(lane);
-    [[maybe_unused]] HadMfma H;
+    [[maybe_unused]] HadMfmaWords H{};
     if constexpr (MF)
     {
-        H = had_mfma_operands(lane);
+        H = had_mfma_words(lane);   // (two words: the 8-VGPR operands cost the rotated-input form a wave per SIMD)
         if constexpr ((HAD & HAD_IN) != 0)
         {
             // x = the producing projection's output rotation, every lane of the wave taking part
@@ -428,14 +444,11 @@ __device__ __forceinline__ void rms_finish(const RmsArgs& a, int64_t row, int ti
             #pragma unroll
             for (int k = 0; k < MAXV; ++k)
             {
-                const int cp = cp0 + k * nt;
-                post[k] = cp < nc ? a.hxpost : nullptr;
-                col[k] = (int64_t)cp * 8;
-                L.xv[k] = mfma_permute(L.xv[k], lane);
+                const int c = c0 + k * nt;
+                post[k] = c < nc ? a.hxpost : nullptr;
+                col[k] = (int64_t)c * 8;
             }
             output_rotations_mfma<MAXV>(H, L.xv, post, col, lane);
-            #pragma unroll
-            for (int k = 0; k < MAXV; ++k) L.xv[k] = mfma_permute(L.xv[k], lane);
         }
     }
     // Pass 1: residual update and sum of squares.  The row is then cached in its narrowest exact
@@ -473,6 +486,9 @@ __device__ __forceinline__ void rms_finish(const RmsArgs& a, int64_t row, int ti
         // Pass 2 with the matrix-core transforms: the f16 norm output of every live chunk (zeros past the
         // row), then each consumer's had_r_128 with its pre-scale, every lane of the wave taking part.
         static_assert((HAD & HAD_OUT) != 0 && YT::code == DT_F16 && !SPLIT, "the Hadamard outputs follow an f16 norm");
+        // With one chunk per lane nothing is waited for after the first store (see RowRegs): the weight is used
+        // before it.  Longer rows go chunk by chunk, the residual's store first.
+        static_assert(WM == W_EARLY, "Hadamard rows take the weight with their loads");
         #pragma unroll
         for (int k = 0; k < MAXV; ++k)
         {
@@ -483,47 +499,46 @@ __device__ __forceinline__ void rms_finish(const RmsArgs& a, int64_t row, int ti
             yv.a = u32x4{ 0u, 0u, 0u, 0u };
             if (live)
             {
-                if constexpr (WM == W_LATE)
-                {
-                    if (a.w) L.wv[k] = prefetch_w8(a.w, a.wt, wofs + e);
-                }
+                auto norm = [&] { yv = rms_out8<XT, YT, RT, MODE>(a, e, wofs, cache[k], L.rv[k], L.wv[k], rmf); };
+                if constexpr (MAXV == 1) norm();
                 if constexpr (kDeferResidual<MODE, RT>)
                 {
+#ifdef EXL3R_TUNING
                     if (a.r_cached) store8c<RT>(rrow, e, cache[k]);
-                    else store8<RT>(rrow, e, cache[k]);
+                    else
+#endif
+                        store8<RT>(rrow, e, cache[k]);
                 }
-                yv = rms_out8<XT, YT, RT, MODE>(a, e, wofs, cache[k], L.rv[k], L.wv[k], rmf);
+                if constexpr (MAXV != 1) norm();
                 if (a.y) store8<YT>(yrow, e, yv);
             }
-            // the consumers' transforms of this chunk (at most 4) in the matrix-core placement, their
-            // MFMAs issued together, each result moved back to its lane for the store
-            const TF16::Vec yp = mfma_permute(yv, lane);
-            const int cp = cp0 + k * nt;
-            const bool plive = cp < nc;
-            const int64_t ep = (int64_t)cp * 8;
+            // the consumers' transforms of this chunk (at most 4), their MFMAs issued together
             // (in pairs: four results at once would hold 32 more VGPRs and cost a wave per SIMD)
             #pragma unroll
             for (int i0 = 0; i0 < 4; i0 += 2)
             {
                 if (i0 >= a.nh) break;
                 MfmaOut m[2];
+                TF16::Vec v[2];
                 #pragma unroll
                 for (int d = 0; d < 2; ++d)
                 {
                     const int i = i0 + d;
-                    if (i < a.nh)
+                    v[d] = yv;
+                    if (i < a.nh && a.hpre[i])   // (lanes past the row hold zeros)
                     {
-                        TF16::Vec v = yp;
-                        if (plive && a.hpre[i])
-                        {
-                            const TF16::Vec p = load8<TF16>(a.hpre[i], pre_row(a, row) + ep);
-                            #pragma unroll
-                            for (int q = 0; q < 4; ++q) v.a[q] = hmul2(v.a[q], p.a[q]);
-                        }
-                        m[d] = had128_mfma_issue(H, v);
+                        u32x4 p;
+                        if constexpr (kRowPre<HAD, MAXV> > 0) p = L.pv[k][i];
+                        else p = load8<TF16>(a.hpre[i], pre_row(a, row) + (live ? e : 0)).a;
+                        #pragma unroll
+                        for (int q = 0; q < 4; ++q) v[d].a[q] = hmul2(v[d].a[q], (uint32_t)p[q]);
                     }
-                    else
-                        m[d] = MfmaOut{};
+                }
+                if (i0 + 1 < a.nh) had128_mfma_issue_w(H, v[0], v[1], m[0], m[1]);
+                else
+                {
+                    had128_mfma_issue_w(H, v[0], m[0]);
+                    m[1] = MfmaOut{};
                 }
                 mfma_wait_all(m);
                 #pragma unroll
@@ -534,37 +549,69 @@ __device__ __forceinline__ void rms_finish(const RmsArgs& a, int64_t row, int ti
                     {
                         float f[8];
                         had128_mfma_finish(m[d], f, lane, a.hr);
-                        const TF16::Vec o = mfma_permute(pack8<TF16>(f), lane);
-                        if (live) store8<TF16>((char*)a.hout[i] + row * a.ldh * 2, e, o);
+                        if (live) store8<TF16>((char*)a.hout[i] + row * a.ldh * 2, e, pack8<TF16>(f));
                     }
                 }
             }
         }
         return;
     }
-    // Pass 2: scale, weight, round once, store.
+    if constexpr (HAD == 0)
+    {
+        // Pass 2: scale, weight, round once; then the stores, none of them before the last weight has arrived
+        // (see RowRegs: a weight waited for after a store waits for the store too).
+        if constexpr (WM == W_LATE)
+        {
+            #pragma unroll
+            for (int k = 0; k < MAXV; ++k)
+            {
+                const int c = tid + k * nt;
+                if (c < nc && a.w) L.wv[k] = prefetch_w8<SPLIT>(a.w, a.wt, wofs + chunk_elem<SPLIT>(c));
+            }
+        }
+        typename YT::Vec ys[MAXV];
+        #pragma unroll
+        for (int k = 0; k < MAXV; ++k)
+        {
+            const int c = tid + k * nt;
+            if (c < nc)
+                ys[k] = rms_out8<XT, YT, RT, MODE, SPLIT>(a, chunk_elem<SPLIT>(c), wofs, cache[k], L.rv[k], L.wv[k], rmf);
+        }
+        #pragma unroll
+        for (int k = 0; k < MAXV; ++k)
+        {
+            const int c = tid + k * nt;
+            const int64_t e = chunk_elem<SPLIT>(c);
+            if (c < nc)
+            {
+                if constexpr (kDeferResidual<MODE, RT>)
+                {
+                    if constexpr (SPLIT) store8_split<RT>(rrow, e, cache[k]);
+                    else store8<RT>(rrow, e, cache[k]);
+                }
+                if constexpr (SPLIT) store8_split<YT>(yrow, e, ys[k]);
+                else store8<YT>(yrow, e, ys[k]);
+            }
+        }
+        return;
+    }
+    // Pass 2 with the butterfly: scale, weight, round once, rotate, store.
     #pragma unroll
     for (int k = 0; k < MAXV; ++k)
     {
         const int c = tid + k * nt;
         if (c < nc)
         {
-            const int64_t e = chunk_elem<SPLIT>(c);
-            if constexpr (WM == W_LATE)
-            {
-                if (a.w) L.wv[k] = prefetch_w8<SPLIT>(a.w, a.wt, wofs + e);
-            }
+            const int64_t e = (int64_t)c * 8;
             if constexpr (kDeferResidual<MODE, RT>)
             {
-                if constexpr (SPLIT) store8_split<RT>(rrow, e, cache[k]);
-                else if constexpr (HAD != 0)
-                {
-                    if (a.r_cached) store8c<RT>(rrow, e, cache[k]);
-                    else store8<RT>(rrow, e, cache[k]);
-                }
-                else store8<RT>(rrow, e, cache[k]);
+#ifdef EXL3R_TUNING
+                if (a.r_cached) store8c<RT>(rrow, e, cache[k]);
+                else
+#endif
+                    store8<RT>(rrow, e, cache[k]);
             }
-            rms_chunk2<XT, YT, RT, MODE, HAD, SPLIT>(a, row, yrow, e, wofs, cache[k], L.rv[k], L.wv[k], rmf);
+            rms_chunk2<XT, YT, RT, MODE, HAD>(a, row, yrow, e, wofs, cache[k], L.rv[k], L.wv[k], rmf);
         }
     }
 }
@@ -588,7 +635,7 @@ __global__ __launch_bounds__(1024) void k_rms_norm(RmsArgs a)
     __shared__ ACC red[16];
     rms_fetch_args(a);
     const int64_t row = a.row0 + blockIdx.x;
-    RowRegs<XT, RT, MAXV> L;
+    RowRegs<XT, RT, MAXV, kRowPre<HAD, MAXV>> L;
     rms_load<XT, RT, MAXV, MODE, SPLIT, HAD>(a, row, threadIdx.x, blockDim.x, WM == W_EARLY, L);
     rms_finish<XT, YT, RT, MAXV, MODE, HAD, WM, SPLIT, ACC>(a, row, threadIdx.x, blockDim.x, L, red);
 }
@@ -901,6 +948,18 @@ inline RmsShape rms_shape(int nc, int64_t rows, int mode, int had, bool wide = f
         return sh;
     }
 #endif
+    // Matrix-core Hadamard rows: one chunk per lane while 1024 lanes cover the row, the pre-scales held beside it
+    // (f16 x / f32 r, three outputs, rotated input, us for 1 / 2 / 4 chunks per lane: [4096, 5120] 69.0 / 73.4 /
+    // 76.1, [8192, 5120] 131.1 / 137.5 / 139.3, [4096, 2560] 35.6 / 38.0 / 39.4, [4096, 4096] 53.4 / 55.4 / 60.0).
+    // Two chunks per lane halve a row's waves, so where they let the launch run in one round of resident
+    // workgroups, with some room, and one chunk does not, they win ([1200, 5120] 20.1 against 25.8, [1100, 5120]
+    // 19.6 / 23.7; at 1500 of 1536 rows a round 30.9 / 29.6).
+    if ((had & HAD_MFMA) && thr(1) <= 1024)
+    {
+        const int64_t round1 = (int64_t)(2048 / thr(1)) * device_cus(), round2 = (int64_t)(2048 / thr(2)) * device_cus();
+        if (rows > round1 && rows <= round2 - round2 / 8) return { 2, thr(2), W_EARLY };
+        return { 1, thr(1), W_EARLY };
+    }
     if (rows > 1024 && mode == RMS_RES_IN && !had)
     {
         if (nc <= 512) return { 1, thr(1), W_LATE };

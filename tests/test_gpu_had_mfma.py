@@ -257,6 +257,14 @@ def test_norm_had_partial_spans():
     run_norm(5, 128, F16, None, n_out=1, rotate_x=True, seed=65)
 
 
+@pytest.mark.parametrize("rows,dim", [(1, 128), (768, 5120), (769, 5120), (1345, 5120), (2100, 640), (70, 8320)])
+def test_norm_had_launch_shapes(rows, dim):
+    """The ends of the launch rule: one chunk per lane with the pre-scales held, two chunks where those rows run in
+    one round (769 to 1344 of 5120), rows past 1024 lanes (8320), and widths that end inside a 512-element span."""
+    run_norm(rows, dim, F16, F32, n_out=4, with_y=False, rotate_x=True, seed=rows)
+    run_norm(rows, dim, BF16, None, n_out=1, with_y=True, cb=1.0, seed=rows + 1)
+
+
 @pytest.mark.parametrize("act,rot", [("silu", (True, True)), ("gelu", (False, False))])
 def test_strided_rows_padding_untouched(act, rot):
     """Strided x, y, z and out (row strides past cols): the matrix-core kernel reaches every row through a
