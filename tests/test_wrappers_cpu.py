@@ -120,3 +120,17 @@ def test_well_formed_table_passes_validation(op):
     fails only where the launch needs a GPU."""
     with pytest.raises(RuntimeError, match="GPU"):
         call(op, INV, torch.zeros((3, 64, 2), dtype=torch.float32))
+
+
+def test_native_wrappers_decline_what_is_not_theirs():
+    """CPU tensors, wrong argument counts and types are left to the Python wrapper (None), nothing is launched."""
+    _lib.load()
+    assert _lib.fast is not None, "exl3r/_fast.so is not built"
+    x = torch.zeros((2, 128), dtype=F16)
+    assert _lib.fast.rms_norm(x, None, x, 1e-6, 0.0, 1.0, None) is None
+    assert _lib.fast.rms_norm(x, None, x) is None
+    assert _lib.fast.rms_norm(1, 2, 3, 4, 5, 6, 7) is None
+    assert _lib.fast.sample(x, x, 0, None, None) is None
+    with _lib.tuned():
+        assert _lib.fast is None            # the sweep build's own entry points are called
+    assert _lib.fast is not None
