@@ -557,7 +557,7 @@ def argmax_sample(logits, ids, max_logit=0, stream=None):
 def gumbel_sample(logits, ids, max_logit=0, random=0, stream=None):
     """ids[i] = argmax of logits[i, :max_logit] + Gumbel(0, 1) noise of (random, i, column): a draw from
     softmax(logits[i, :max_logit]) (src/ffi.rs:526-530)."""
-    if _lib.fast is not None:
+    if _lib.fast is not None and random is not None:   # None asks the native call for the argmax
         rc = _lib.fast.sample(logits, ids, max_logit, random, stream)
         if rc is not None:
             check(rc)

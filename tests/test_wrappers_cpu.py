@@ -134,3 +134,18 @@ def test_native_wrappers_decline_what_is_not_theirs():
     with _lib.tuned():
         assert _lib.fast is None            # the sweep build's own entry points are called
     assert _lib.fast is not None
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="would launch on host tensors")
+def test_a_draw_without_a_seed_never_becomes_the_argmax(monkeypatch):
+    """random=None is the native call's argmax; gumbel_sample refuses it as it refuses any other non-number."""
+    _lib.load()
+
+    class Native:
+        @staticmethod
+        def sample(*args):
+            raise AssertionError(f"native call made: {args[3]!r}")
+
+    monkeypatch.setattr(_lib, "fast", Native)
+    with pytest.raises(TypeError):
+        exl3r.ffi.gumbel_sample(torch.zeros((2, 128)), torch.zeros(2, dtype=torch.int64), random=None)
