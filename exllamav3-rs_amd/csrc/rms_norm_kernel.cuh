@@ -678,20 +678,28 @@ __global__ __launch_bounds__(1024) void k_rms_norm_pipe(RmsArgs a)
 }
 
 // Short rows (at most 64 chunks of 8): LPR lanes per row (a power of two covering dim / 8), one
-// chunk per lane, 256 / LPR rows per workgroup and RPL rows per lane in flight.  The row sum is a
+// chunk per lane, one-wave workgroups of 64 / LPR rows and RPL rows per lane in flight.  The row sum is a
 // DPP butterfly inside the LPR-lane group -- no LDS, no barrier -- so a 128-element head row costs
 // 16 lanes instead of a workgroup.
+// HBM-bound with a short life per wave (one item), so what stands before its first load counts: the arguments
+// arrive in one scalar batch (they came in three dependent ones) and there is no grid walk, whose strides and
+// 64-bit products were set up first and held registers (78 VGPRs, 6 waves per SIMD; now 43, 8 waves).  Gated norm
+// with the o_proj rotation, [131072, 128] bf16 x / f32 g: 27.1 -> 25.1 us, 5.35 TB/s.
 // HAD_MFMA (rows of one 128-element block, one f16 output): a wave's 4 rows are one span of
 // had128_mfma's placement -- row = lane bits 2-3, chunk = lane bits 0, 1, 4, 5 -- so the row sum runs
 // over lanes xor 1, 2, 16 and 32, which groups it as the 16-lane butterfly does (quads, pairs of quads,
 // then the two pairs), the same bits.
 template <class XT, class YT, class RT, int LPR, int RPL, int MODE, int HAD = 0>
-__global__ __launch_bounds__(256) void k_rms_rows(RmsArgs a)
+__global__ __launch_bounds__(64) void k_rms_rows(RmsArgs a)
 {
     static_assert(MODE != RMS_GATHER, "gathered rows take the workgroup kernel");
     constexpr bool MF = (HAD & HAD_MFMA) != 0;
     static_assert(!MF || (LPR == 16 && (HAD & HAD_OUT) != 0), "matrix-core rows: one block each, an output");
-    const int SLOTS = (int)blockDim.x / LPR;   // row slots of the workgroup
+    constexpr int SLOTS = 64 / LPR;            // row slots of the workgroup, one wave
+    rms_fetch_args(a);
+    asm volatile("" : : "s"(a.rows), "s"(a.gact), "s"(a.gfirst), "s"(a.w_groups));
+    if constexpr ((HAD & HAD_OUT) != 0)
+        asm volatile("" : : "s"(a.hpre[0]), "s"(a.hpre_rows), "s"(a.hout[0]), "s"(a.ldh), "s"(a.hr));
     const int l64 = threadIdx.x & 63;
     const int lane = MF ? (l64 & 3) | ((l64 >> 2) & 12) : (int)threadIdx.x % LPR;
     const int slot = MF ? (int)(threadIdx.x >> 6) * 4 + ((l64 >> 2) & 3) : (int)threadIdx.x / LPR;
@@ -699,7 +707,7 @@ __global__ __launch_bounds__(256) void k_rms_rows(RmsArgs a)
     const int64_t e = (int64_t)lane * 8;
     [[maybe_unused]] HadMfmaWords hw{};
     if constexpr (MF) hw = had_mfma_words(l64);
-    for (int64_t r0 = (int64_t)blockIdx.x * SLOTS * RPL; r0 < a.rows; r0 += (int64_t)gridDim.x * SLOTS * RPL)
+    const int64_t r0 = a.row0 + (int64_t)blockIdx.x * (SLOTS * RPL);
     {
         typename XT::Vec xv[RPL];
         typename RT::Vec rv[RPL];
@@ -792,20 +800,27 @@ void launch_rms_rows(const RmsArgs& a, hipStream_t s)
     const int nc = a.dim >> 3;
     auto go = [&](auto L) {
         constexpr int LPR = decltype(L)::value;
-        // One-wave workgroups (same process, both orders, us for 64 / 256 lanes at [131072, 128]: gated
-        // norm 24.8 / 25.2, with the o_proj rotation on the matrix cores 28.6 / 29.5, butterfly 28.9 / 29.1).
+        // One-wave workgroups (when the kernel walked its grid, same process, both orders, us for 64 / 256 lanes at
+        // [131072, 128]: gated norm 24.8 / 25.2, with the o_proj rotation on the matrix cores 28.6 / 29.5,
+        // butterfly 28.9 / 29.1).
         constexpr int kThreads = 64;
         constexpr int SLOTS = kThreads / LPR;
         const int tuned = tuning().rms_rows_rpl;
-        // One row per lane: at 62 VGPRs (f32 gate) 8 waves per SIMD keep the loads in flight.  Measured
-        // on MI355X, gated norm [131072, 128] bf16 x / f32 g / f16 y: 1 row per lane 25.2 us, 2 rows
-        // 30.6 us, 4 rows (156 VGPRs) 33.4 us; a workgroup per row 63 us.
+        // One row per lane.  us at 1 / 2 / 4, bf16 x / f16 y: [131072, 128] f32 gate 23.3 / 25.5 / 29.3, with the
+        // rotation 25.2 / 27.8 / 30.7, bf16 gate 19.5 / 21.3 / 25.5; [4000, 128] f32 gate 3.2 / 4.2 / 6.7.  (A
+        // workgroup per row: 63 at [131072, 128].)
         const int rpl = (tuned == 1 || tuned == 2 || tuned == 4) ? tuned : 1;
-        int64_t blocks = (a.rows + (int64_t)SLOTS * rpl - 1) / ((int64_t)SLOTS * rpl);
-        if (blocks > kMaxGridX) blocks = kMaxGridX;
-        if (rpl == 4) launch(k_rms_rows<XT, YT, RT, LPR, 4, MODE, HAD>, (unsigned)blocks, kThreads, 0, s, a);
-        else if (rpl == 2) launch(k_rms_rows<XT, YT, RT, LPR, 2, MODE, HAD>, (unsigned)blocks, kThreads, 0, s, a);
-        else launch(k_rms_rows<XT, YT, RT, LPR, 1, MODE, HAD>, (unsigned)blocks, kThreads, 0, s, a);
+        // More rows than kMaxGridX workgroups hold go out in several launches (row0: the first row of each).
+        const int64_t per = (int64_t)SLOTS * rpl;
+        RmsArgs b = a;
+        for (b.row0 = 0; b.row0 < a.rows; b.row0 += kMaxGridX * per)
+        {
+            int64_t blocks = (a.rows - b.row0 + per - 1) / per;
+            if (blocks > kMaxGridX) blocks = kMaxGridX;
+            if (rpl == 4) launch(k_rms_rows<XT, YT, RT, LPR, 4, MODE, HAD>, (unsigned)blocks, kThreads, 0, s, b);
+            else if (rpl == 2) launch(k_rms_rows<XT, YT, RT, LPR, 2, MODE, HAD>, (unsigned)blocks, kThreads, 0, s, b);
+            else launch(k_rms_rows<XT, YT, RT, LPR, 1, MODE, HAD>, (unsigned)blocks, kThreads, 0, s, b);
+        }
     };
     if constexpr ((HAD & HAD_MFMA) != 0)
         go(std::integral_constant<int, 16>{});   // rows of one block (the caller checks dim == 128)

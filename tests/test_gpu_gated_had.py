@@ -121,3 +121,26 @@ def test_zero_rows_and_errors():
         ffi.gated_rms_norm_had(x, None, g, torch.empty((4, 128), device="cuda", dtype=torch.float16), 1e-6,
                                pre_rows=3)
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("dim,rows", [(8, 8 * 2 ** 20 + 5), (128, 4 * 2 ** 20 + 3)])
+def test_more_rows_than_one_grid(dim, rows):
+    """Short rows beyond the workgroups of one launch (2**20, of 8 or 4 rows) go out in several: every row as in calls
+    that one launch holds, bit for bit, with the weight groups and pre-scale rows counted from the call's first row."""
+    x = torch.randn((rows, dim), device="cuda", dtype=torch.bfloat16)
+    g = torch.randn((rows, dim), device="cuda", dtype=torch.bfloat16)
+    cut = rows // 2 // 6 * 6
+    w = torch.randn((3 * dim,), device="cuda")
+    pre = suh(dim, 1) if dim == 128 else None
+
+    def call(a, b):
+        out = torch.full((b - a, dim), 7.0, device="cuda", dtype=torch.float16)
+        if dim == 128:
+            ffi.gated_rms_norm_had(x[a:b], w, g[a:b], out, 1e-6, pre, w_groups=3)
+        else:
+            ffi.gated_rms_norm(x[a:b], w, out, g[a:b], 1e-6, w_groups=3)
+        return out.view(torch.int16)
+
+    whole = call(0, rows)
+    assert torch.equal(whole[:cut], call(0, cut))
+    assert torch.equal(whole[cut:], call(cut, rows))
