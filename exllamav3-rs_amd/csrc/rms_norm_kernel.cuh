@@ -708,89 +708,87 @@ __global__ __launch_bounds__(64) void k_rms_rows(RmsArgs a)
     [[maybe_unused]] HadMfmaWords hw{};
     if constexpr (MF) hw = had_mfma_words(l64);
     const int64_t r0 = a.row0 + (int64_t)blockIdx.x * (SLOTS * RPL);
+    typename XT::Vec xv[RPL];
+    typename RT::Vec rv[RPL];
+    u32x4 wv[RPL];
+    [[maybe_unused]] TF16::Vec pv[RPL];     // HAD_OUT: the row's pre-scale chunk, fetched with its loads
+    bool act[RPL];
+    #pragma unroll
+    for (int i = 0; i < RPL; ++i)
     {
-        typename XT::Vec xv[RPL];
-        typename RT::Vec rv[RPL];
-        u32x4 wv[RPL];
-        [[maybe_unused]] TF16::Vec pv[RPL];     // HAD_OUT: the row's pre-scale chunk, fetched with its loads
-        bool act[RPL];
-        #pragma unroll
-        for (int i = 0; i < RPL; ++i)
+        const int64_t row = r0 + (int64_t)i * SLOTS + slot;
+        act[i] = lane_ok && row < a.rows;
+        if (act[i])
         {
-            const int64_t row = r0 + (int64_t)i * SLOTS + slot;
-            act[i] = lane_ok && row < a.rows;
+            xv[i] = load8s<XT>((const char*)a.x + row * a.ldx * XT::bytes, e);
+            if constexpr (MODE == RMS_RES_IN || MODE == RMS_GATED)
+                rv[i] = load8s<RT>((const char*)a.r + row * a.ldr * RT::bytes, e);
+            if (a.w) wv[i] = prefetch_w8(a.w, a.wt, weight_row<MODE>(a, row) + e);
+            if constexpr ((HAD & HAD_OUT) != 0)
+                if (a.hpre[0]) pv[i] = load8<TF16>(a.hpre[0], pre_row(a, row) + e);
+        }
+    }
+    #pragma unroll
+    for (int i = 0; i < RPL; ++i)
+    {
+        const int64_t row = r0 + (int64_t)i * SLOTS + slot;
+        double ss = 0.0;
+        typename RmsCache<XT, RT, MODE>::Vec cv;
+        if (act[i]) cv = rms_chunk1<XT, RT, MODE>(a, (char*)a.r + row * a.ldr * RT::bytes, e, true, xv[i], rv[i], ss);
+        if constexpr (MF)
+        {
+            ss += dpp64<DPP_QUAD_XOR1>(ss);
+            ss += dpp64<DPP_QUAD_XOR2>(ss);
+            ss = sum_xor32(sum_xor16(ss));
+        }
+        else
+            ss = group_sum64<LPR>(ss);
+        const float rmf = rms_factor(ss, a.dim, a.eps) * a.cs;
+        if constexpr (MF)
+        {
+            // The f16 norm output and its pre-scale product (zeros in the rows past the end, whose
+            // lanes still take part in the MFMAs), the transform, then the stores of live rows.
+            TF16::Vec v = {};
             if (act[i])
             {
-                xv[i] = load8s<XT>((const char*)a.x + row * a.ldx * XT::bytes, e);
-                if constexpr (MODE == RMS_RES_IN || MODE == RMS_GATED)
-                    rv[i] = load8s<RT>((const char*)a.r + row * a.ldr * RT::bytes, e);
-                if (a.w) wv[i] = prefetch_w8(a.w, a.wt, weight_row<MODE>(a, row) + e);
-                if constexpr ((HAD & HAD_OUT) != 0)
-                    if (a.hpre[0]) pv[i] = load8<TF16>(a.hpre[0], pre_row(a, row) + e);
+                v = rms_out8<XT, YT, RT, MODE, false>(a, e, weight_row<MODE>(a, row), cv, rv[i], wv[i], rmf);
+                if (a.y) store8<YT>((char*)a.y + row * a.ldy * YT::bytes, e, v);
+                if (a.hpre[0])
+                {
+                    #pragma unroll
+                    for (int q = 0; q < 4; ++q) v.a[q] = hmul2(v.a[q], pv[i].a[q]);
+                }
             }
+            MfmaOut m;
+            had128_mfma_issue_w(hw, v, m);
+            mfma_wait(m);
+            float f[8];
+            had128_mfma_finish(m, f, l64, a.hr);
+            if (act[i]) store8<TF16>((char*)a.hout[0] + row * a.ldh * 2, e, pack8<TF16>(f));
         }
-        #pragma unroll
-        for (int i = 0; i < RPL; ++i)
+        else if constexpr ((HAD & HAD_OUT) != 0)
         {
-            const int64_t row = r0 + (int64_t)i * SLOTS + slot;
-            double ss = 0.0;
-            typename RmsCache<XT, RT, MODE>::Vec cv;
-            if (act[i]) cv = rms_chunk1<XT, RT, MODE>(a, (char*)a.r + row * a.ldr * RT::bytes, e, true, xv[i], rv[i], ss);
-            if constexpr (MF)
+            // the butterfly on the row's 16-lane block groups (one output), as rms_chunk2 does it
+            static_assert(YT::code == DT_F16, "the Hadamard prologue follows an f16 norm output");
+            if (act[i])
             {
-                ss += dpp64<DPP_QUAD_XOR1>(ss);
-                ss += dpp64<DPP_QUAD_XOR2>(ss);
-                ss = sum_xor32(sum_xor16(ss));
-            }
-            else
-                ss = group_sum64<LPR>(ss);
-            const float rmf = rms_factor(ss, a.dim, a.eps) * a.cs;
-            if constexpr (MF)
-            {
-                // The f16 norm output and its pre-scale product (zeros in the rows past the end, whose
-                // lanes still take part in the MFMAs), the transform, then the stores of live rows.
-                TF16::Vec v = {};
-                if (act[i])
+                TF16::Vec v = rms_out8<XT, YT, RT, MODE, false>(a, e, weight_row<MODE>(a, row), cv, rv[i], wv[i], rmf);
+                if (a.y) store8<YT>((char*)a.y + row * a.ldy * YT::bytes, e, v);
+                if (a.hpre[0])
                 {
-                    v = rms_out8<XT, YT, RT, MODE, false>(a, e, weight_row<MODE>(a, row), cv, rv[i], wv[i], rmf);
-                    if (a.y) store8<YT>((char*)a.y + row * a.ldy * YT::bytes, e, v);
-                    if (a.hpre[0])
-                    {
-                        #pragma unroll
-                        for (int q = 0; q < 4; ++q) v.a[q] = hmul2(v.a[q], pv[i].a[q]);
-                    }
+                    #pragma unroll
+                    for (int q = 0; q < 4; ++q) v.a[q] = hmul2(v.a[q], pv[i].a[q]);
                 }
-                MfmaOut m;
-                had128_mfma_issue_w(hw, v, m);
-                mfma_wait(m);
-                float f[8];
-                had128_mfma_finish(m, f, l64, a.hr);
-                if (act[i]) store8<TF16>((char*)a.hout[0] + row * a.ldh * 2, e, pack8<TF16>(f));
+                with_carried<true>(zero_lane16(v), a.hr, [&](auto C) {
+                    float f[8];
+                    butterfly128_f16<decltype(C)::value>(v, f, lane & 15, a.hr);
+                    store8<TF16>((char*)a.hout[0] + row * a.ldh * 2, e, pack8<TF16>(f));
+                });
             }
-            else if constexpr ((HAD & HAD_OUT) != 0)
-            {
-                // the butterfly on the row's 16-lane block groups (one output), as rms_chunk2 does it
-                static_assert(YT::code == DT_F16, "the Hadamard prologue follows an f16 norm output");
-                if (act[i])
-                {
-                    TF16::Vec v = rms_out8<XT, YT, RT, MODE, false>(a, e, weight_row<MODE>(a, row), cv, rv[i], wv[i], rmf);
-                    if (a.y) store8<YT>((char*)a.y + row * a.ldy * YT::bytes, e, v);
-                    if (a.hpre[0])
-                    {
-                        #pragma unroll
-                        for (int q = 0; q < 4; ++q) v.a[q] = hmul2(v.a[q], pv[i].a[q]);
-                    }
-                    with_carried<true>(zero_lane16(v), a.hr, [&](auto C) {
-                        float f[8];
-                        butterfly128_f16<decltype(C)::value>(v, f, lane & 15, a.hr);
-                        store8<TF16>((char*)a.hout[0] + row * a.ldh * 2, e, pack8<TF16>(f));
-                    });
-                }
-            }
-            else if (act[i])
-                rms_chunk2<XT, YT, RT, MODE, HAD>(a, row, (char*)a.y + row * a.ldy * YT::bytes, e,
-                                                      weight_row<MODE>(a, row), cv, rv[i], wv[i], rmf);
         }
+        else if (act[i])
+            rms_chunk2<XT, YT, RT, MODE, HAD>(a, row, (char*)a.y + row * a.ldy * YT::bytes, e,
+                                                  weight_row<MODE>(a, row), cv, rv[i], wv[i], rmf);
     }
 }
 
