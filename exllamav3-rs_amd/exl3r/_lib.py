@@ -5,6 +5,7 @@ missing -- there is no fallback implementation of any op."""
 import contextlib
 import ctypes
 import os
+import sys
 
 _PKG_ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 LIB_DIR = os.path.join(_PKG_ROOT, "lib")
@@ -124,8 +125,8 @@ NAIVE_PROTOTYPES = {
 _lib = None
 _naive = None
 _tune = None
-# The native wrappers (exl3r/_fast.so over the product library; None until load(), where it is not built, and
-# inside tuned()).  ffi.py offers them every call and makes the ones that they decline itself.
+# The native wrappers (exl3r/_fast.so over the product library; None until load(), where it is not built or built
+# for another torch or interpreter, and inside tuned()).  ffi.py offers them every call and makes the ones that they decline itself.
 fast = None
 _fast_names = ("exl3r_rms_norm", "exl3r_rms_norm_res_in", "exl3r_silu_mul", "exl3r_gelu_mul", "exl3r_mul_sigmoid",
                "exl3r_gated_rms_norm", "exl3r_gated_rms_norm_had", "exl3r_rope", "exl3r_rope_table", "exl3r_rope_qg",
@@ -135,9 +136,11 @@ _fast_names = ("exl3r_rms_norm", "exl3r_rms_norm_res_in", "exl3r_silu_mul", "exl
 
 def _bind_fast(lib):
     try:
-        import torch  # noqa: F401  (its libraries are the module's)
+        import torch  # (its libraries are the module's)
         from . import _fast
     except ImportError:
+        return None
+    if getattr(_fast, "built_for", None) != f"{torch.__version__} {sys.implementation.cache_tag}":
         return None
     for name in _fast_names:
         if not _fast.bind(name, ctypes.cast(getattr(lib, name), ctypes.c_void_p).value):

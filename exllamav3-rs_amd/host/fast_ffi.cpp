@@ -529,4 +529,11 @@ PyModuleDef module = { PyModuleDef_HEAD_INIT, "_fast", nullptr, -1, methods, nul
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__fast() { return PyModule_Create(&module); }
+// built_for: the torch and the interpreter it is compiled against, whose C++ and C ABIs it uses; the loader compares
+// them with the ones that run.
+PyMODINIT_FUNC PyInit__fast()
+{
+    PyObject* m = PyModule_Create(&module);
+    if (m && PyModule_AddStringConstant(m, "built_for", EXL3R_BUILT_FOR)) Py_CLEAR(m);
+    return m;
+}

@@ -45,3 +45,21 @@ def test_make_without_a_rocm_torch(tree, tmp_path, torch_of_cpu):
     assert r.returncode == 0, r.stderr
     assert "skipped" in r.stdout
     assert not (tree / "exl3r" / "_fast.so").exists()
+
+
+def test_module_follows_the_torch_it_is_built_for(tree, tmp_path):
+    """Another torch version or interpreter tag builds the module again; the same ones do not."""
+    (tree / "exl3r").mkdir()
+    so, run = tree / "exl3r" / "_fast.so", no_torch(tmp_path, True)
+    (tmp_path / "site" / "torch" / "include" / "c10" / "hip").mkdir(parents=True)
+    (tmp_path / "site" / "torch" / "include" / "c10" / "hip" / "HIPStream.h").write_text("")
+    compiler = tmp_path / "cxx"
+    compiler.write_text("#!/bin/sh\necho \"$@\" >> %s\ntouch exl3r/_fast.so\n" % (tmp_path / "built"))
+    compiler.chmod(0o755)
+    built = lambda: (tmp_path / "built").read_text().splitlines()
+    for version, builds in (("2.0.0", 1), ("2.0.0", 1), ("2.1.0", 2), ("2.1.0", 2)):
+        (tmp_path / "site" / "torch" / "version.py").write_text(f"__version__ = {version!r}\n")
+        r = make(tree, run, f"CXX={compiler}", "exl3r/_fast.so")
+        assert r.returncode == 0 and so.exists(), r.stderr
+        assert len(built()) == builds
+        assert f'-DEXL3R_BUILT_FOR="{version} {sys.implementation.cache_tag}"' in built()[-1]

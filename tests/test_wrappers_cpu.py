@@ -136,6 +136,14 @@ def test_native_wrappers_decline_what_is_not_theirs():
     assert _lib.fast is not None
 
 
+def test_native_wrappers_of_another_torch_are_not_used(monkeypatch):
+    """The module is compiled against one torch's C++ classes and one interpreter; it is used with no other."""
+    lib = _lib.load()
+    assert _lib._bind_fast(lib) is not None
+    monkeypatch.setattr(torch, "__version__", "1.0.0")
+    assert _lib._bind_fast(lib) is None
+
+
 @pytest.mark.skipif(torch.cuda.is_available(), reason="would launch on host tensors")
 def test_a_draw_without_a_seed_never_becomes_the_argmax(monkeypatch):
     """random=None is the native call's argmax; gumbel_sample refuses it as it refuses any other non-number."""
