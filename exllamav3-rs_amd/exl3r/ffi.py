@@ -155,7 +155,7 @@ def gated_rms_norm_had(x, w, g, out, eps, pre_scale=None, y=None, constant_bias=
     gate_act)."""
     if _lib.fast is not None:
         rc = _lib.fast.gated_rms_norm_had(x, w, g, out, eps, pre_scale, y, constant_bias, w_groups, gate_first,
-                                          gate_act | (HAD_EXACT if exact else 0), had_scale, pre_rows, stream)
+                                          int(gate_act) | (HAD_EXACT if exact else 0), had_scale, pre_rows, stream)
         if rc is not None:
             check(rc)
             return

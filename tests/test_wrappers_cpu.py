@@ -157,3 +157,22 @@ def test_a_draw_without_a_seed_never_becomes_the_argmax(monkeypatch):
     monkeypatch.setattr(_lib, "fast", Native)
     with pytest.raises(TypeError):
         exl3r.ffi.gumbel_sample(torch.zeros((2, 128)), torch.zeros(2, dtype=torch.int64), random=None)
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="would launch on host tensors")
+def test_gate_act_of_any_number(monkeypatch):
+    """gated_rms_norm_had takes gate_act through int(), also in the native call's flags."""
+    _lib.load()
+    seen = []
+
+    class Native:
+        @staticmethod
+        def gated_rms_norm_had(*args):
+            seen.append(args[10])
+            return 0
+
+    monkeypatch.setattr(_lib, "fast", Native)
+    x = torch.zeros((2, 128), dtype=F16)
+    for act in (1, 1.0, True, torch.tensor(1)):
+        ffi.gated_rms_norm_had(x, None, x, x, 1e-6, gate_act=act, exact=True)
+    assert seen == [1 | _lib.HAD_EXACT] * 4
