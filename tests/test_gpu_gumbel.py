@@ -153,3 +153,79 @@ def test_sample_masks_of_the_lowest_value(rows):
         x[1::2, 5000:5010] = np.linspace(-2, 2, 10)
         x[1::2, 12294] = 1.0
         run_sample(to_dev(orc.to_bits(x, dt), dt), dt, 94)
+
+
+LOWEST = {F16: -65504.0, BF16: -3.3895313892515355e38, F32: -3.4028234663852886e38}
+
+
+@pytest.mark.parametrize("rows,vocab", [(3, 30001), (16, 30000), (400, 12295)])
+@pytest.mark.parametrize("dt", [F16, BF16, F32])
+def test_sample_masked_slices(rows, vocab, dt):
+    """Rows with slices that hold no live logit: -inf, -1e9 and lowest-value masks with a few live columns or none,
+    a NaN or +inf somewhere, on the sliced kernels (three launches and one) and the row kernel."""
+    rng = np.random.default_rng(rows)
+    for low in (-np.inf, -1e9 if dt != F16 else -6e4, LOWEST[dt]):
+        x = np.full((rows, vocab), low, np.float32)
+        for r in range(rows):
+            if r % 4:
+                x[r, rng.integers(0, vocab, 5)] = rng.normal(0, 3, 5)
+        x[0, vocab - 1] = (np.nan, np.inf, 1.0)[rows % 3]
+        x[2, [7, vocab - 3]] = np.nan
+        x[1, vocab // 2:] = -np.inf
+        dev = to_dev(orc.to_bits(x, dt), dt)
+        got = run_sample(dev, dt, 95)
+        if rows < 384:
+            ids = torch.empty(rows, dtype=torch.int64, device="cuda")
+            ws = torch.zeros(ffi.sample_workspace_bytes(), dtype=torch.uint8, device="cuda")
+            ffi.gumbel_sample_ws(dev, ids, ws, 0, 95)
+            torch.cuda.synchronize()
+            assert np.array_equal(ids.cpu().numpy(), got)
+
+
+@pytest.mark.parametrize("rows", [16, 400])
+def test_sample_where_the_noise_is_absorbed(rows):
+    """Logits about the size (0x1.1p29) from which half the float spacing is more than any noise, on both sides of
+    it, each row a few neighbouring floats of one size and sign: below it the noise still decides between them."""
+    rng = np.random.default_rng(5)
+    size = np.float32(2.0) ** rng.uniform(26, 33, (rows, 1)).astype(np.float32)
+    size[:8, 0] = [2.0 ** 28, 2.0 ** 29, 570425344.0, np.nextafter(np.float32(570425344.0), 0), 2.0 ** 30, 1e9, 2.0 ** 31, 6e8]
+    x = size.view(np.uint32) + rng.integers(-2, 3, (rows, 10250)).astype(np.uint32)
+    x = x.astype(np.uint32).view(np.float32) * np.where(np.arange(rows) % 2, 1.0, -1.0)[:, None].astype(np.float32)
+    run_sample(to_dev(np.ascontiguousarray(x), F32), F32, 96)
+
+
+def graph_us(fn, n=10):
+    fn()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        for _ in range(n):
+            fn()
+    best = math.inf
+    for _ in range(5):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        graph.replay()
+        a.record()
+        graph.replay()
+        b.record()
+        torch.cuda.synchronize()
+        best = min(best, a.elapsed_time(b) * 1e3 / n)
+    return best
+
+
+@pytest.mark.parametrize("rows", [16, 64])
+def test_masked_draws_take_no_longer_than_live_ones(rows):
+    """A top-k mask leaves most slices of a row without a live logit; they need no noise (us per draw of 151936 f32
+    logits; with every masked candidate evaluated one by one, 20.3 against 9.3 at 16 rows and 27 against 14.3 at
+    64).  The factor is for the clock."""
+    live = dev_normal((rows, 151936), 0, 3, F32, 97)
+    keep = torch.topk(live, 50, dim=1).indices
+    ids = torch.empty(rows, dtype=torch.int64, device="cuda")
+    us = {None: graph_us(lambda: ffi.gumbel_sample(live, ids, 0, 3))}
+    for low in (-math.inf, -1e9, LOWEST[F32]):
+        x = torch.full_like(live, low).scatter_(1, keep, live.gather(1, keep))
+        us[low] = graph_us(lambda: ffi.gumbel_sample(x, ids, 0, 3))
+    x = live.clone()
+    x[:, 1000] = math.nan
+    us["nan"] = graph_us(lambda: ffi.gumbel_sample(x, ids, 0, 3))
+    assert max(us.values()) < 1.25 * us[None], us
