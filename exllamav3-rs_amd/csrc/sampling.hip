@@ -499,6 +499,15 @@ __device__ __forceinline__ uint64_t slice_lane_key(const ArgArgs& a, int64_t row
     return lb.key();
 }
 
+// First element of the workgroup's slice.  Only a draw's slices have a length that the kernel does not know: with a
+// length from memory the argmax of four chunks per lane needs more than 96 VGPRs, a wave per SIMD less.
+template <int UNROLL, bool GUMBEL>
+__device__ __forceinline__ int64_t slice_start(const ArgArgs& a)
+{
+    if constexpr (GUMBEL) return (int64_t)blockIdx.x * a.slice;
+    else return (int64_t)blockIdx.x * UNROLL * 2048;
+}
+
 // A workgroup of 256 lanes reduces a slice of UNROLL * 2048 elements (UNROLL chunks of 8 per lane in
 // flight) to one key, so a row takes only vocab / slice atomics: same-address atomics from many
 // workgroups (and XCDs) serialize.
@@ -508,7 +517,7 @@ __global__ __launch_bounds__(256) void k_argmax(ArgArgs a)
     __shared__ uint64_t part[4];
     __shared__ float wmax[4];
     const int tid = threadIdx.x;
-    const int64_t start = (int64_t)blockIdx.x * a.slice;
+    const int64_t start = slice_start<UNROLL, GUMBEL>(a);
     for (int64_t row = blockIdx.y; row < a.rows; row += gridDim.y)
     {
         uint64_t best = wave_max_u64(slice_lane_key<IT, VEC, UNROLL, GUMBEL>(a, row, start, tid, wmax));
@@ -540,7 +549,7 @@ __global__ __launch_bounds__(256) void k_argmax_ws(ArgArgs a, uint32_t* count, u
     __shared__ float wmax[4];
     const int tid = threadIdx.x;
     const uint32_t slices = gridDim.x;
-    const int64_t start = (int64_t)blockIdx.x * a.slice;
+    const int64_t start = slice_start<UNROLL, GUMBEL>(a);
     for (int64_t row = blockIdx.y; row < a.rows; row += gridDim.y)
     {
         uint64_t best = wave_max_u64(slice_lane_key<IT, VEC, UNROLL, GUMBEL>(a, row, start, tid, wmax));

@@ -1,0 +1,78 @@
+"""Registers and scratch of kernels in the built library, from the metadata that the compiler writes beside each: a
+kernel whose waves per SIMD or whose scratch its speed depends on stays within what it was measured with."""
+import os
+import re
+import shutil
+import struct
+import subprocess
+
+import pytest
+
+from exl3r import _lib
+
+msgpack = pytest.importorskip("msgpack")
+
+BUNDLE, ELF_NOTE, AMDGPU_METADATA = b"__CLANG_OFFLOAD_BUNDLE__", 7, 32
+
+
+def notes(elf):
+    """The descriptors of an ELF64 image's notes, by type."""
+    shoff, = struct.unpack_from("<Q", elf, 0x28)
+    entry, count, _ = struct.unpack_from("<HHH", elf, 0x3A)
+    for i in range(count):
+        kind, = struct.unpack_from("<I", elf, shoff + i * entry + 4)
+        at, size = struct.unpack_from("<QQ", elf, shoff + i * entry + 0x18)
+        end = at + size
+        while kind == ELF_NOTE and at < end:
+            name, desc, note = struct.unpack_from("<III", elf, at)
+            at += 12 + (name + 3) // 4 * 4
+            yield note, elf[at:at + desc]
+            at += (desc + 3) // 4 * 4
+
+
+@pytest.fixture(scope="module")
+def kernels():
+    """Demangled name -> metadata of every kernel of the product library."""
+    with open(_lib.LIB_PATH, "rb") as f:
+        image = f.read()
+    found, at = {}, image.find(BUNDLE)
+    while at >= 0:
+        count, = struct.unpack_from("<Q", image, at + 24)
+        p = at + 32
+        for _ in range(count):
+            off, size, length = struct.unpack_from("<QQQ", image, p)
+            target = image[p + 24:p + 24 + length]
+            p += 24 + length
+            if b"gfx950" in target and size:
+                for kind, desc in notes(image[at + off:at + off + size]):
+                    if kind == AMDGPU_METADATA:
+                        for k in msgpack.unpackb(desc, strict_map_key=False)["amdhsa.kernels"]:
+                            found[k[".name"]] = k
+        at = image.find(BUNDLE, at + 24)
+    if not shutil.which("c++filt"):
+        pytest.skip("no c++filt")
+    names = sorted(found)
+    out = subprocess.run(["c++filt"], input="\n".join(names), capture_output=True, text=True, check=True).stdout.split("\n")
+    return {d.replace("exl3r::", ""): found[n] for d, n in zip(out, names)}
+
+
+def matching(kernels, pattern):
+    hits = {n: k for n, k in kernels.items() if re.search(pattern, n)}
+    assert hits, pattern
+    return hits
+
+
+# pattern of the instances, VGPRs at most (96: 5 waves per SIMD, 80: 6, 64: 8), spilled VGPRs and scratch bytes per
+# lane at most
+LIMITS = [
+    # argmax, four chunks of aligned logits in flight
+    (r"void k_argmax(_ws)?<\w+, true, 4, false>", 96, 0, 0),
+]
+
+
+@pytest.mark.parametrize("pattern,vgprs,spills,scratch", LIMITS)
+def test_resources(kernels, pattern, vgprs, spills, scratch):
+    over = {n: (k[".vgpr_count"], k[".vgpr_spill_count"], k[".private_segment_fixed_size"])
+            for n, k in matching(kernels, pattern).items()
+            if k[".vgpr_count"] > vgprs or k[".vgpr_spill_count"] > spills or k[".private_segment_fixed_size"] > scratch}
+    assert not over, over
