@@ -16,9 +16,9 @@
 // Philox4x32-10 is the published generator of Salmon, Moraes, Dror and Shaw ("Parallel random
 // numbers: as easy as 1, 2, 3", SC 2011).
 //
-// Layout, few rows (decode): a row is cut into slices of 2048 or 8192 elements, a 256-lane
-// workgroup per slice (grid (slices, rows)), so a single decode row of 152k logits still spreads over
-// ~75 CUs.  From 128 rows (argmax) or 384 rows (Gumbel draw): a workgroup of 512 or 1024 lanes per
+// Layout, few rows (decode): a row is cut into slices of 2048 or 8192 elements (argmax) or 2048 to 10240
+// (draw), a 256-lane workgroup per slice (grid (slices, rows)), so a single decode row of 152k logits still
+// spreads over ~75 CUs.  From 128 rows (argmax) or 384 rows (Gumbel draw): a workgroup of 512 or 1024 lanes per
 // row, the index written directly.  Each lane keeps its
 // best candidate as one 64-bit key -- an order-preserving image of the value in the high word, the
 // complement of the index in the low word -- so "larger key" is exactly "larger value, then lower
@@ -282,7 +282,7 @@ __device__ __forceinline__ typename IT::Vec load_chunk(const void* base, int64_t
 // than any noise (-2.9 .. 16.7), so x + g is x for every candidate that can win, and with NaN or +inf about, x + g
 // is NaN or +inf where x is.  The slice's draw is then its logits' argmax, the first index where all are -inf.  (us in
 // a HIP graph, 16 / 64 rows of 151936 f32 logits, live 9.3 / 14.3, all but 50 columns of a row -inf 9.0 / 14.0, -1e9
-// 10.3 / 15.3, a NaN in every row 9.5 / 16.4; one by one with their noise 20.2 / 26.9, 20.2 / 25.1 and 21 / 25.3.)
+// 11.0 / 15.3, a NaN in every row 9.5 / 16.4; one by one with their noise 20.2 / 26.9, 20.2 / 25.1 and 21 / 25.3.)
 // 64 rows of 151936 f32 logits took 22.0 us with
 // every candidate exact, bound by VALU issue, and take 14.7 (three launches, ~13 us of host time from Python); 1024 rows 247 -> 122.5 us (5.1 TB/s).
 constexpr float kRankErr = 1e-5f;
@@ -444,17 +444,42 @@ __device__ __forceinline__ uint64_t gumbel_lane_key(const ArgArgs& a, int64_t ro
 }
 
 // One lane's best candidate over its UNROLL chunks of the slice starting at `start` of `row`.  A chunk crossing
-// n is read element by element.  GUMBEL: the workgroup's largest rank (wmax: one LDS slot per wave) decides
-// which candidates are evaluated; every lane of the workgroup must get here.
+// n is read element by element.  GUMBEL: a slice of one chunk per lane (UNROLL 1) evaluates them all; in a longer
+// one (any UNROLL above) the workgroup's largest rank (wmax: one LDS slot per wave) decides which, and every lane of
+// the workgroup must get here.
 template <class IT, bool VEC, int UNROLL, bool GUMBEL>
 __device__ __forceinline__ uint64_t slice_lane_key(const ArgArgs& a, int64_t row, int64_t start, int tid, float* wmax)
 {
     const char* base = a.x + row * a.ld;
     LaneBest lb;
-    if constexpr (GUMBEL)
+    if constexpr (GUMBEL && UNROLL > 1)
     {
         const int64_t end = start + a.slice;
         return gumbel_lane_key<IT, VEC, 256>(a, row, start, end < a.n ? end : a.n, tid, wmax);
+    }
+    if constexpr (GUMBEL)
+    {
+        #pragma clang fp contract(off)
+        const int64_t c = start + tid * 8;
+        if (c >= a.n) return 0;
+        typename IT::Vec v{};
+        if (c + 8 <= a.n) v = load_chunk<IT, VEC>(base, c);
+        float g[8];
+        gumbel8(a.seed, row, c, g);
+        if (__builtin_expect(c + 8 <= a.n, 1))
+        {
+            float x[8];
+            unpack8<IT>(v, x);
+            #pragma unroll
+            for (int j = 0; j < 8; ++j) lb.consider(x[j] + g[j], c + j);
+        }
+        else
+        {
+            #pragma unroll
+            for (int j = 0; j < 7; ++j)
+                if (c + j < a.n) lb.consider(load1(base, IT::code, c + j) + g[j], c + j);
+        }
+        return lb.key();
     }
     typename IT::Vec v[UNROLL];
     #pragma unroll
@@ -499,16 +524,16 @@ __device__ __forceinline__ uint64_t slice_lane_key(const ArgArgs& a, int64_t row
     return lb.key();
 }
 
-// First element of the workgroup's slice.  Only a draw's slices have a length that the kernel does not know: with a
-// length from memory the argmax of four chunks per lane needs more than 96 VGPRs, a wave per SIMD less.
+// First element of the workgroup's slice.  Only a draw's longer slices have a length that the kernel does not know:
+// with a length from memory the argmax of four chunks per lane needs more than 96 VGPRs, a wave per SIMD less.
 template <int UNROLL, bool GUMBEL>
 __device__ __forceinline__ int64_t slice_start(const ArgArgs& a)
 {
-    if constexpr (GUMBEL) return (int64_t)blockIdx.x * a.slice;
+    if constexpr (GUMBEL && UNROLL > 1) return (int64_t)blockIdx.x * a.slice;
     else return (int64_t)blockIdx.x * UNROLL * 2048;
 }
 
-// A workgroup of 256 lanes reduces a slice of UNROLL * 2048 elements (UNROLL chunks of 8 per lane in
+// A workgroup of 256 lanes reduces a slice (argmax: UNROLL * 2048 elements, UNROLL chunks of 8 per lane in
 // flight) to one key, so a row takes only vocab / slice atomics: same-address atomics from many
 // workgroups (and XCDs) serialize.
 template <class IT, bool VEC, int UNROLL, bool GUMBEL>
@@ -726,6 +751,28 @@ constexpr size_t kWsBytes = kCountBytes + kWsMaxRows * 8;
 // few rows take 2048-element slices so the row still spreads over enough CUs.
 inline int slice_unroll(int64_t rows) { return rows >= 16 ? 4 : 1; }
 
+// Chunks of 8 logits per lane of a draw's slices.  A slice costs its workgroup a reduction, the winner's evaluation
+// and an atomic on the row's word, so slices are long, up to 10240 elements, while they leave half the CUs a
+// workgroup.  One chunk per lane evaluates its candidates as they come: ranking them first costs a small draw a second
+// read of the winner's chunk (1 row of 32000 f32 logits 6.47 us ranked, 6.26 as they come).  MI355X, HIP graph, f32,
+// us for 1 / 2 / 3 / 4 / 5 / 6 / 8 chunks (1: as they come), three launches:
+//     1 x 151936   6.84 / 6.97 / 7.32 / 7.80 / 8.20 / 8.61 / 9.40
+//     8 x 151936  13.25 / 9.85 / 9.14 / 9.09 / 9.55 / 10.3 / 11.3
+//    16 x 32000    7.75 / 7.31 / 7.52 / 7.94 / 8.70 / 9.08 / 10.9
+//    16 x 151936  16.4 / 11.5 / 10.2 / 10.6 / 10.1 / 10.6 / 11.7
+//    64 x 32000   10.6 / 8.63 / 9.09 / 9.04 / 9.66 / 10.4 / 11.8
+//    64 x 151936  28.8 / 19.1 / 16.2 / 15.5 / 15.0 / 16.0 / 15.6
+//   256 x 151936  66.6 / 42.4 / 37.0 / 35.6 / 35.6 / 36.4 / 37.1
+// Over 1 to 383 rows of 32000 to 262144 logits, f16 and f32, with and without the workspace, it is 4% from the best
+// of them on average, 24% at most (one slice of a few elements left over; few rows in the workspace); 2048-element
+// slices below 16 rows and 10240 from there on were 13%, 150% at most.
+inline int draw_chunks(int64_t n, int64_t rows)
+{
+    for (int k = 5; k > 1; --k)
+        if (rows * ((n + k * 2048 - 1) / (k * 2048)) >= device_cus() / 2) return k;
+    return 1;
+}
+
 struct Workspace
 {
     void* base;      // nullptr: the three-launch path (ids as the reduction slot)
@@ -814,13 +861,9 @@ int sample_entry(const char* op, const void* logits, int dtype, int64_t rows, in
         });
         return launch_status(op);
     }
-    const int unroll = GUMBEL ? 1 : slice_unroll(rows);   // (chunks in flight per lane; the draw's loop has its own)
-    int64_t slice = (int64_t)unroll * 2048;
-    // The draw's slices are longer: each costs its workgroup a reduction, the winner's evaluation and an atomic
-    // (us for slices of 2048 / 4096 / 6144 / 8192 / 10240 / 12288 / 16384 f32 logits, 151936 a row, with the
-    // ~13 us of three launches from Python as the floor: 16 rows 16.4 / 13 / 13 / 13 / 13 / 13 / 13, 64 rows
-    // 28.1 / 19.1 / 16.8 / 15.7 / 15.2 / 16.1 / 15.8, 256 rows 62.6 / 42.8 / 37.4 / 37.6 / 35.8 / 36.5 / 38.3).
-    if (GUMBEL && rows >= 16) slice = 5 * 2048;
+    int unroll = slice_unroll(rows);
+    if (GUMBEL) unroll = tu.sample_slice > 0 ? tu.sample_slice : draw_chunks(n, rows);
+    const int64_t slice = (int64_t)unroll * 2048;
     a.slice = slice;
     const dim3 grid((unsigned)((n + slice - 1) / slice), (unsigned)rows);
     if (ws.scratch)
@@ -841,10 +884,10 @@ int sample_entry(const char* op, const void* logits, int dtype, int64_t rows, in
         uint64_t* part = (uint64_t*)((char*)ws.base + kCountBytes);
         with_float_type(dtype, [&](auto T) {
             using Ty = decltype(T);
-            if (!GUMBEL && unroll == 4)
+            if (unroll > 1)
             {
-                if (vec) launch(k_argmax_ws<Ty, true, GUMBEL ? 1 : 4, GUMBEL>, grid, 256, 0, s, a, count, part);
-                else launch(k_argmax_ws<Ty, false, GUMBEL ? 1 : 4, GUMBEL>, grid, 256, 0, s, a, count, part);
+                if (vec) launch(k_argmax_ws<Ty, true, 4, GUMBEL>, grid, 256, 0, s, a, count, part);
+                else launch(k_argmax_ws<Ty, false, 4, GUMBEL>, grid, 256, 0, s, a, count, part);
             }
             else
             {
@@ -858,10 +901,10 @@ int sample_entry(const char* op, const void* logits, int dtype, int64_t rows, in
     launch(k_argmax_clear, small, 256, 0, s, a.ids, rows);
     with_float_type(dtype, [&](auto T) {
         using Ty = decltype(T);
-        if (!GUMBEL && unroll == 4)
+        if (unroll > 1)
         {
-            if (vec) launch(k_argmax<Ty, true, GUMBEL ? 1 : 4, GUMBEL>, grid, 256, 0, s, a);
-            else launch(k_argmax<Ty, false, GUMBEL ? 1 : 4, GUMBEL>, grid, 256, 0, s, a);
+            if (vec) launch(k_argmax<Ty, true, 4, GUMBEL>, grid, 256, 0, s, a);
+            else launch(k_argmax<Ty, false, 4, GUMBEL>, grid, 256, 0, s, a);
         }
         else
         {

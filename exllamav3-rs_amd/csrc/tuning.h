@@ -34,6 +34,8 @@ EXL3R_API void exl3r_tune_rope_nx_run(int run);
 EXL3R_API void exl3r_tune_rope_ss32(int on);
 /* argmax / Gumbel sampling: rows from which a workgroup owns a whole row (0: 512), and its lanes (256, 512, 1024) */
 EXL3R_API void exl3r_tune_sample(int rows_min, int threads);
+/* Gumbel draw, sliced kernels: chunks of 8 logits per lane, so 2048 times as many logits per slice (0 auto) */
+EXL3R_API void exl3r_tune_sample_slice(int chunks);
 /* Hadamard: 128-blocks per 16-lane group (1, 2, 4; 0 auto) */
 EXL3R_API void exl3r_tune_had(int blocks_per_group);
 /* matrix-core Hadamard kernels: spans (act-mul: rows of a span) per wave in flight (1, 2, 4; 0 auto),

@@ -104,6 +104,7 @@ TUNE_PROTOTYPES = {
     "exl3r_tune_rope_nx_run": (None, [_i]),
     "exl3r_tune_rope_ss32": (None, [_i]),
     "exl3r_tune_sample": (None, [_i, _i]),
+    "exl3r_tune_sample_slice": (None, [_i]),
     "exl3r_tune_had": (None, [_i]),
     "exl3r_tune_had_mfma": (None, [_i, _i]),
     "exl3r_tune_had_threads": (None, [_i]),
@@ -208,6 +209,7 @@ def tuned():
         lib.exl3r_tune_rope_nx_run(0)
         lib.exl3r_tune_rope_ss32(0)
         lib.exl3r_tune_sample(0, 0)
+        lib.exl3r_tune_sample_slice(0)
         lib.exl3r_tune_had(0)
         lib.exl3r_tune_had_mfma(0, 0)
         lib.exl3r_tune_had_threads(0)

@@ -229,3 +229,27 @@ def test_masked_draws_take_no_longer_than_live_ones(rows):
     x[:, 1000] = math.nan
     us["nan"] = graph_us(lambda: ffi.gumbel_sample(x, ids, 0, 3))
     assert max(us.values()) < 1.25 * us[None], us
+
+
+@pytest.mark.parametrize("chunks", [1, 2, 3, 4, 5])
+@pytest.mark.parametrize("vocab", [1, 2048, 10240, 12289, 30001])
+def test_sample_slice_lengths(chunks, vocab):
+    """Every slice length, whole and cut short by the row's end, aligned rows and rows off by one element, and a last
+    slice of one element."""
+    from exl3r import _lib
+    with _lib.tuned() as lib:
+        lib.exl3r_tune_sample_slice(chunks)
+        for dt in (F16, F32):
+            x = dev_normal((5, vocab + 1), 0, 3, dt, 98)
+            run_sample(x[:, :vocab].contiguous(), dt, 99)
+            run_sample(x[:, 1:], dt, 99)
+            run_sample(x, dt, 99, max(1, vocab - 4))
+
+
+def test_fewer_rows_take_no_longer():
+    """The slices follow the work of the whole draw: 15 rows (15.4 us in slices of 2048 logits) against 16 (9.3 in
+    longer ones), and few rows of a small vocabulary against as many of a large one."""
+    ids = torch.empty(16, dtype=torch.int64, device="cuda")
+    x = dev_normal((16, 151936), 0, 3, F32, 100)
+    few, many = (graph_us(lambda: ffi.gumbel_sample(x[:n], ids[:n], 0, 3)) for n in (15, 16))
+    assert few < 1.15 * many, (few, many)
