@@ -29,6 +29,9 @@
 
 #include "abi.hpp"
 #include "common.cuh"
+#ifdef EXL3R_TUNING
+#include "tuning.h"
+#endif
 
 namespace exl3r {
 
@@ -272,7 +275,7 @@ __device__ __forceinline__ typename IT::Vec load_chunk(const void* base, int64_t
 // log_f32's noise for the candidates that come within a bound of the best rank, one as a rule.
 //
 // b = x - ln2 log2(-log2 u) is the candidate x + g less the constant -ln ln 2.  Over all 2^23 values of u
-// the noise part differs from g by less than kRankErr (by 1.6e-6 at most, measured), and forming b and
+// the noise part differs from g by less than kRankErr (by 1.58e-6 at most: k_rank_error walks them), and forming b and
 // x + g rounds each by at most 2^-24 of its size, so with m the largest b, a candidate with
 // b < m - (2 kRankErr + 2^-20 |m|) is below the one that has b = m: |b| <= 2 |m| leaves 3 * 2^-23 |m| for the
 // roundings, and a larger |b| (b far below m) is more than |b| / 2 away.  The best candidate, and any that
@@ -309,6 +312,18 @@ __device__ __forceinline__ float wave_max_nan(float v)
     const auto q = __builtin_amdgcn_permlane32_swap(w, w, false, false);
     return max_nan(__builtin_bit_cast(float, (uint32_t)q[0]), __builtin_bit_cast(float, (uint32_t)q[1]));
 }
+
+#ifdef EXL3R_TUNING
+// out[0]: the largest distance of the ranked noise (with the constant -ln ln 2 that it leaves out) from the exact one
+// over all 2^23 values of u, a lane each; out[1]: the bound that the draw allows it.
+__global__ __launch_bounds__(256) void k_rank_error(float* out)
+{
+    const uint32_t bits = (blockIdx.x * 256 + threadIdx.x) << 9;
+    const double d = (double)gumbel_rank(0.0f, bits) + 0.36651292058166432701 - (double)gumbel_of_bits(bits);
+    atomicMax((unsigned*)out, __builtin_bit_cast(uint32_t, (float)fabs(d)));
+    if (bits == 0) out[1] = kRankErr;
+}
+#endif
 
 // The chunk's 8 logits (-inf past the row), from the loaded vector or, for a chunk that crosses n, one by one.
 template <class IT>
@@ -917,6 +932,16 @@ int sample_entry(const char* op, const void* logits, int dtype, int64_t rows, in
 }
 
 }  // namespace
+
+#ifdef EXL3R_TUNING
+extern "C" int exl3r_tune_gumbel_rank_error(float* out, void* stream)
+{
+    begin_call();
+    launch(k_argmax_clear, 1, 256, 0, (hipStream_t)stream, (uint64_t*)out, 1);
+    launch(k_rank_error, (1u << 23) / 256, 256, 0, (hipStream_t)stream, out);
+    return launch_status("exl3r_tune_gumbel_rank_error");
+}
+#endif
 
 extern "C" int exl3r_argmax_sample_noalloc(const void* logits, int dtype, int64_t rows, int64_t vocab, int64_t ld,
                                            int max_logit, int64_t* ids, void* stream)

@@ -36,6 +36,9 @@ EXL3R_API void exl3r_tune_rope_ss32(int on);
 EXL3R_API void exl3r_tune_sample(int rows_min, int threads);
 /* Gumbel draw, sliced kernels: chunks of 8 logits per lane, so 2048 times as many logits per slice (0 auto) */
 EXL3R_API void exl3r_tune_sample_slice(int chunks);
+/* out[0]: the largest distance of the noise that ranks a draw's candidates from their exact noise over all 2^23
+ * uniforms, out[1]: the bound that the draw's exactness rests on (out: two floats on the device, 8-byte aligned) */
+EXL3R_API int exl3r_tune_gumbel_rank_error(float* out, void* stream);
 /* Hadamard: 128-blocks per 16-lane group (1, 2, 4; 0 auto) */
 EXL3R_API void exl3r_tune_had(int blocks_per_group);
 /* matrix-core Hadamard kernels: spans (act-mul: rows of a span) per wave in flight (1, 2, 4; 0 auto),

@@ -105,6 +105,7 @@ TUNE_PROTOTYPES = {
     "exl3r_tune_rope_ss32": (None, [_i]),
     "exl3r_tune_sample": (None, [_i, _i]),
     "exl3r_tune_sample_slice": (None, [_i]),
+    "exl3r_tune_gumbel_rank_error": (_i, [_vp, _vp]),
     "exl3r_tune_had": (None, [_i]),
     "exl3r_tune_had_mfma": (None, [_i, _i]),
     "exl3r_tune_had_threads": (None, [_i]),

@@ -253,3 +253,14 @@ def test_fewer_rows_take_no_longer():
     x = dev_normal((16, 151936), 0, 3, F32, 100)
     few, many = (graph_us(lambda: ffi.gumbel_sample(x[:n], ids[:n], 0, 3)) for n in (15, 16))
     assert few < 1.15 * many, (few, many)
+
+
+def test_rank_error_over_every_uniform():
+    """The draw is exact as long as the hardware's log2 keeps the ranked noise within its bound of the exact noise,
+    for every one of the 2^23 values of u."""
+    from exl3r import _lib
+    out = torch.full((2,), math.nan, device="cuda")
+    _lib.check(_lib.load_tune().exl3r_tune_gumbel_rank_error(out.data_ptr(), torch.cuda.current_stream().cuda_stream))
+    err, bound = out.tolist()
+    print(f"largest error {err:.3e}, bound {bound:.1e}")
+    assert 0.0 < err < bound / 2
