@@ -86,11 +86,12 @@ __device__ __forceinline__ int first_chunk(int tid)
 // When a row's weight chunks are fetched (a launch-shape choice: the results are the same bits).
 //   W_EARLY: with the row's HBM loads, so the L2 fetch overlaps them (latency-bound launches);
 //   W_MID:   after pass 1, so the fetch overlaps the row reduction;
+//   W_FIRST: as W_MID, and pass 2 forms every output before its first store (see rms_finish);
 //   W_LATE:  chunk by chunk in pass 2, after the reduction.
 // Streaming launches fetch it late: the row then holds no weight registers while its HBM loads are in
 // flight (MI355X, [8192, 5120]: bf16 residual norm 56.3 us early -> 54.9 late; f16 x / f32 r / f16 y
 // 93.6 -> 88.6; plain bf16 norm 31.5 -> 30.7 mid).
-enum { W_EARLY = 0, W_MID = 1, W_LATE = 2 };
+enum { W_EARLY = 0, W_MID = 1, W_LATE = 2, W_FIRST = 3 };
 
 // RMS_GATED gate activation in fp32.
 __device__ __forceinline__ float gate_act(int gact, float g) { return gact ? act_f<ACT_SIGMOID>(g) : act_f<ACT_SILU>(g); }
@@ -466,7 +467,7 @@ __device__ __forceinline__ void rms_finish(const RmsArgs& a, int64_t row, int ti
     }
 
     const int64_t wofs = weight_row<MODE>(a, row);
-    if constexpr (WM == W_MID)
+    if constexpr (WM == W_MID || WM == W_FIRST)
     {
         #pragma unroll
         for (int k = 0; k < MAXV; ++k)
@@ -556,19 +557,11 @@ __device__ __forceinline__ void rms_finish(const RmsArgs& a, int64_t row, int ti
         }
         return;
     }
-    if constexpr (HAD == 0)
+    // Pass 2: scale, weight, round once, store.  Two orders, the same bits.
+    if constexpr (HAD == 0 && (WM == W_FIRST || (WM == W_EARLY && MAXV == 1)))
     {
-        // Pass 2: scale, weight, round once; then the stores, none of them before the last weight has arrived
-        // (see RowRegs: a weight waited for after a store waits for the store too).
-        if constexpr (WM == W_LATE)
-        {
-            #pragma unroll
-            for (int k = 0; k < MAXV; ++k)
-            {
-                const int c = tid + k * nt;
-                if (c < nc && a.w) L.wv[k] = prefetch_w8<SPLIT>(a.w, a.wt, wofs + chunk_elem<SPLIT>(c));
-            }
-        }
+        // Weights first: every output is formed before the first store, so no weight is waited for behind a store
+        // (see RowRegs).
         typename YT::Vec ys[MAXV];
         #pragma unroll
         for (int k = 0; k < MAXV; ++k)
@@ -595,23 +588,38 @@ __device__ __forceinline__ void rms_finish(const RmsArgs& a, int64_t row, int ti
         }
         return;
     }
-    // Pass 2 with the butterfly: scale, weight, round once, rotate, store.
+    // Chunk by chunk, the residual's store ahead of the chunk's norm: the stores start sooner and one output is held
+    // at a time (eight held at once spill).  us, chunk by chunk / weights first:
+    //   one chunk per lane, early weights (up to 1024 rows): residual norm [1024, 5120] f16 x / f32 r 13.4 / 13.2, f16
+    //     9.8 / 9.6, [256, 8192] f32 r 5.5 / 5.4, f32 x and y [1024, 5120] 10.0 / 9.8
+    //   plain streaming norms: [8192, 5120] f16 30.2 / 29.2, bf16 29.0 / 28.5, [8192, 1024] f16 7.9 / 7.6
+    //   late weights: bf16 residual [8192, 5120] 53.3 / 53.7, [8192, 1024] 11.6 / 12.2, [2048, 16384] 44.1 / 45.9
+    //   split chunks: f16 x / f32 r [4096, 8192] 64.9 / 66.8, [2048, 16384] 68.1 / 69.9, f32 throughout [8192, 5120]
+    //     107.6 / 110.3; on 128 lanes, [8192, 1024], 16.1 / 15.6
+    //   more chunks per lane (wide rows), f32 to f32 [256, 16384] 9.7 / 12.7, [1500, 32768] 86.2 / 152.4, f16 x /
+    //     f32 r / f32 y [1500, 40960] 242.6 / 319.2
+    // With Hadamard outputs (the butterfly): scale, weight, round once, rotate, store.
     #pragma unroll
     for (int k = 0; k < MAXV; ++k)
     {
         const int c = tid + k * nt;
         if (c < nc)
         {
-            const int64_t e = (int64_t)c * 8;
+            const int64_t e = chunk_elem<SPLIT>(c);
+            if constexpr (WM == W_LATE)
+            {
+                if (a.w) L.wv[k] = prefetch_w8<SPLIT>(a.w, a.wt, wofs + e);
+            }
             if constexpr (kDeferResidual<MODE, RT>)
             {
 #ifdef EXL3R_TUNING
-                if (a.r_cached) store8c<RT>(rrow, e, cache[k]);
+                if (HAD != 0 && a.r_cached) store8c<RT>(rrow, e, cache[k]);
                 else
 #endif
-                    store8<RT>(rrow, e, cache[k]);
+                if constexpr (SPLIT) store8_split<RT>(rrow, e, cache[k]);
+                else store8<RT>(rrow, e, cache[k]);
             }
-            rms_chunk2<XT, YT, RT, MODE, HAD>(a, row, yrow, e, wofs, cache[k], L.rv[k], L.wv[k], rmf);
+            rms_chunk2<XT, YT, RT, MODE, HAD, SPLIT>(a, row, yrow, e, wofs, cache[k], L.rv[k], L.wv[k], rmf);
         }
     }
 }
@@ -927,7 +935,10 @@ inline RmsShape rms_shape(int nc, int64_t rows, int mode, int had, bool wide = f
     auto thr = [&](int m) { int t = (nc + m - 1) / m; return ((t + 63) / 64) * 64; };
     auto pick = [&](int m) { return m <= 1 ? 1 : m <= 2 ? 2 : m <= 4 ? 4 : 8; };
     const bool split_ok = !had && (mode == RMS_PLAIN || mode == RMS_RES_IN) && nc % 64 == 0 && nc <= 2048;
-    auto split_shape = [&](int wm) { return RmsShape{ nc <= 1024 ? 1 : 2, nc <= 1024 ? nc : thr(2), wm, true }; };
+    auto split_shape = [&](int wm) {
+        const bool first = wm == W_MID && mode == RMS_RES_IN && nc <= 128;   // (both orders measured at rms_finish)
+        return RmsShape{ nc <= 1024 ? 1 : 2, nc <= 1024 ? nc : thr(2), first ? (int)W_FIRST : wm, true };
+    };
 #ifdef EXL3R_TUNING
     const int split_mode = tuning().rms_split;
     const int split_wm = tuning().rms_split_wm == W_LATE ? W_LATE : W_MID;
@@ -984,7 +995,7 @@ inline RmsShape rms_shape(int nc, int64_t rows, int mode, int had, bool wide = f
     }
     if (rows > 1024)
     {
-        const int wm = !had && mode == RMS_PLAIN ? W_MID : W_EARLY;
+        const int wm = !had && mode == RMS_PLAIN ? W_FIRST : W_EARLY;
         if (thr(1) <= 512) return { 1, thr(1), wm };
         if (thr(2) <= 1024) return { 2, thr(2) > 384 || had ? thr(2) : 384, wm };
     }
@@ -1008,10 +1019,10 @@ void launch_rms_acc(const RmsArgs& a0, const RmsShape& sh, hipStream_t s)
             case 1: launch(k_rms_norm<XT, YT, RT, 1, MODE, HAD, WM, SPLIT, ACC>, grid, sh.threads, 0, s, a); break;
             case 2: launch(k_rms_norm<XT, YT, RT, 2, MODE, HAD, WM, SPLIT, ACC>, grid, sh.threads, 0, s, a); break;
             case 4:
-                if constexpr (!SPLIT) launch(k_rms_norm<XT, YT, RT, 4, MODE, HAD, WM, false, ACC>, grid, sh.threads, 0, s, a);
+                if constexpr (!SPLIT && WM != W_FIRST) launch(k_rms_norm<XT, YT, RT, 4, MODE, HAD, WM, false, ACC>, grid, sh.threads, 0, s, a);
                 break;
             default:
-                if constexpr (!SPLIT) launch(k_rms_norm<XT, YT, RT, 8, MODE, HAD, WM, false, ACC>, grid, sh.threads, 0, s, a);
+                if constexpr (!SPLIT && WM != W_FIRST) launch(k_rms_norm<XT, YT, RT, 8, MODE, HAD, WM, false, ACC>, grid, sh.threads, 0, s, a);
                 break;
         }
     }
@@ -1071,14 +1082,22 @@ void launch_rms_vec(const RmsArgs& a, hipStream_t s)
     {
         if (sh.split)
         {
+#ifdef EXL3R_TUNING
             if (sh.wmode == W_LATE) return launch_rms_wm<XT, YT, RT, MODE, HAD, W_LATE, true>(a, sh, s);
+#endif
+            if constexpr (MODE == RMS_RES_IN)
+                if (sh.wmode == W_FIRST) return launch_rms_wm<XT, YT, RT, MODE, HAD, W_FIRST, true>(a, sh, s);
             return launch_rms_wm<XT, YT, RT, MODE, HAD, W_MID, true>(a, sh, s);
         }
     }
     if constexpr (HAD == 0 && (MODE == RMS_RES_IN || MODE == RMS_PLAIN))
     {
         if (sh.wmode == W_LATE) return launch_rms_wm<XT, YT, RT, MODE, HAD, W_LATE>(a, sh, s);
+#ifdef EXL3R_TUNING
         if (sh.wmode == W_MID) return launch_rms_wm<XT, YT, RT, MODE, HAD, W_MID>(a, sh, s);
+#endif
+        if constexpr (MODE == RMS_PLAIN)
+            if (sh.wmode == W_FIRST) return launch_rms_wm<XT, YT, RT, MODE, HAD, W_FIRST>(a, sh, s);
     }
     launch_rms_wm<XT, YT, RT, MODE, HAD, W_EARLY>(a, sh, s);
 }

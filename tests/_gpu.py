@@ -134,3 +134,23 @@ def assert_head_close(got, exp, hd, what="", rel=2.0 ** -8, max_ulp=2, min_exact
     print(stats)
     assert bad == 0, stats
     assert same.mean() >= min_exact, stats
+
+
+def graph_us(fn, n=10):
+    """Time of one call of fn in a HIP graph of n of them: the best of five replays."""
+    fn()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        for _ in range(n):
+            fn()
+    best = float("inf")
+    for _ in range(5):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        graph.replay()
+        a.record()
+        graph.replay()
+        b.record()
+        torch.cuda.synchronize()
+        best = min(best, a.elapsed_time(b) * 1e3 / n)
+    return best

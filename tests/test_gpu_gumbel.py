@@ -10,7 +10,7 @@ import pytest
 import torch
 
 import exl3r.ffi as ffi
-from _gpu import NTHREADS, TORCH_DT, dev_normal, from_dev, to_dev
+from _gpu import NTHREADS, TORCH_DT, dev_normal, from_dev, graph_us, to_dev
 from oracle import oracle as orc
 
 pytestmark = pytest.mark.gpu
@@ -192,25 +192,6 @@ def test_sample_where_the_noise_is_absorbed(rows):
     x = size.view(np.uint32) + rng.integers(-2, 3, (rows, 10250)).astype(np.uint32)
     x = x.astype(np.uint32).view(np.float32) * np.where(np.arange(rows) % 2, 1.0, -1.0)[:, None].astype(np.float32)
     run_sample(to_dev(np.ascontiguousarray(x), F32), F32, 96)
-
-
-def graph_us(fn, n=10):
-    fn()
-    torch.cuda.synchronize()
-    graph = torch.cuda.CUDAGraph()
-    with torch.cuda.graph(graph):
-        for _ in range(n):
-            fn()
-    best = math.inf
-    for _ in range(5):
-        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-        graph.replay()
-        a.record()
-        graph.replay()
-        b.record()
-        torch.cuda.synchronize()
-        best = min(best, a.elapsed_time(b) * 1e3 / n)
-    return best
 
 
 @pytest.mark.parametrize("rows", [16, 64])

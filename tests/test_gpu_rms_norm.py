@@ -9,7 +9,7 @@ import torch
 
 import exl3r._lib as L
 import exl3r.ffi as ffi
-from _gpu import NTHREADS, assert_bitwise, assert_close_ulp, code_of, dev_normal, from_dev
+from _gpu import NTHREADS, assert_bitwise, assert_close_ulp, code_of, dev_normal, from_dev, graph_us
 from oracle import oracle as orc
 
 pytestmark = pytest.mark.gpu
@@ -179,3 +179,16 @@ def test_split_chunks_strided():
     with L.tuned() as lib:
         lib.exl3r_tune_rms_split(1, 1)
         run_plain(9, 1024, F32, F16, F16, ldx=1024 + 64, ldy=1024 + 128, seed=77)
+
+
+@pytest.mark.parametrize("rows,dim", [(256, 16384), (1500, 32768)])
+def test_wide_f32_rows_store_as_they_go(rows, dim):
+    """f32 rows of several chunks per lane into f32 take about as much longer than into f16 as they move more bytes
+    (4/3): 9.7 against 7.2 us and 86 against 57.  With every output held until the row's last one was formed it was
+    12.7 and 152.  The factor leaves room for the clock."""
+    x, w = dev_normal((rows, dim), 0.0, 1.0, F32, 5), dev_normal((dim,), 1.0, 0.1, F32, 6)
+    us = []
+    for yt in (F32, F16):
+        y = torch.empty((rows, dim), device="cuda", dtype=orc_t(yt))
+        us.append(graph_us(lambda: ffi.rms_norm(x, w, y, 1e-6), 5))
+    assert us[0] < 1.65 * us[1], us

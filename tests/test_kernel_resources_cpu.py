@@ -67,6 +67,12 @@ def matching(kernels, pattern):
 LIMITS = [
     # argmax, four chunks of aligned logits in flight
     (r"void k_argmax(_ws)?<\w+, true, 4, false>", 96, 0, 0),
+    # norms of eight chunks per lane: no row of outputs held beside the row itself
+    (r"void k_rms_norm<(TF16|TBF16), \w+, (TF16|TBF16), 8, 1, 0, 2, false, double>", 98, 0, 0),
+    (r"void k_rms_norm<(TF16|TBF16), TF32, TF32, 8, 1, 0, 2, false, double>", 128, 6, 28),
+    (r"void k_rms_norm<(TF16|TBF16), \w+, TF32, 8, 1, 0, 2, false, double>", 128, 14, 60),
+    (r"void k_rms_norm<TF32, TF32, TF32, 8, 1, 0, 2, false, double>", 128, 56, 164),
+    (r"void k_rms_norm<\w+, \w+, TNone, 8, 0, 0, [02], false, double>", 120, 0, 0),
 ]
 
 
