@@ -70,17 +70,35 @@ constexpr int HAD_OUT = 1;   // rotated f16 outputs, one per projection
 constexpr int HAD_IN = 2;    // x rotated on load
 constexpr int HAD_MFMA = 4;  // the transforms on the matrix cores (had128_mfma)
 
-// The chunk of a row that a thread owns first (its others follow nt chunks apart).  Matrix-core kernels own
-// chunk mfma_chunk(l) of a wave's 64-chunk span in lane l, the transforms' placement, for every load and store
-// of the row: an access of the wave covers the same span either way, in 64-byte (16-bit) or 128-byte (f32)
-// quads.  (Loading rows in lane order and moving them there and back through the lane crossbar, four ds_bpermute
-// per chunk and direction, cost 0.5 us of 78.5.)  Thread counts are multiples of 64, so a wave's chunks are one
-// span of 4 blocks for every k.
-template <int HAD>
+// The matrix-core transforms need chunk mfma_chunk(l) of a wave's 64-chunk span in lane l.  Two ways to have it there:
+// the lane owns that chunk, for every load and store of the row (an access of the wave covers the same span either
+// way, in 64-byte (16-bit) or 128-byte (f32) quads), or the lanes own the chunks in their order and chunks move
+// between the two placements through the lane crossbar (mfma_permute: ds_bpermute, no LDS storage; the permutation is
+// its own inverse).  The first saves the four ds_bpermute per chunk and direction, 0.5 us of 78.5 at [4096, 5120].
+// An f32 residual with two chunks per lane takes the second, and cached residual stores in place of non-temporal
+// ones, which leave its half lines to be merged in L2 (us, owned and non-temporal / lane order and cached, f16 x, three
+// outputs, without and with rotated input: [1200, 5120] 19.7 19.9 / 19.4 18.7, [512, 16384] 27.4 28.0 / 25.3 27.6,
+// [2048, 16384] 105.8 106.4 / 91.7 100.7).  With one chunk per lane, and for 16-bit residuals, cached stores lose
+// ([4096, 5120] f16 residual 47.3 50.7 / 53.0 58.1).
+// Thread counts are multiples of 64, so a wave's chunks are one span of 4 blocks for every k.
+template <class RT, int MAXV, int MODE, int HAD>
+constexpr bool kLaneOrder = (HAD & HAD_MFMA) != 0 && MAXV == 2 && MODE == RMS_RES_IN && RT::code == DT_F32;
+
+// The chunk of a row that a thread owns first (its others follow nt chunks apart).
+template <class RT, int MAXV, int MODE, int HAD>
 __device__ __forceinline__ int first_chunk(int tid)
 {
-    if constexpr ((HAD & HAD_MFMA) != 0) return (tid & ~63) | mfma_chunk(tid & 63);
+    if constexpr ((HAD & HAD_MFMA) != 0 && !kLaneOrder<RT, MAXV, MODE, HAD>) return (tid & ~63) | mfma_chunk(tid & 63);
     else return tid;
+}
+
+__device__ __forceinline__ TF16::Vec mfma_permute(const TF16::Vec& v, int lane)
+{
+    const int src = mfma_chunk(lane) << 2;
+    TF16::Vec o;
+    #pragma unroll
+    for (int q = 0; q < 4; ++q) o.a[q] = (uint32_t)__builtin_amdgcn_ds_bpermute(src, (int)v.a[q]);
+    return o;
 }
 
 // When a row's weight chunks are fetched (a launch-shape choice: the results are the same bits).
@@ -198,7 +216,7 @@ __device__ __forceinline__ void rms_load(const RmsArgs& a, int64_t row, int tid,
     #pragma unroll
     for (int k = 0; k < MAXV; ++k)
     {
-        const int c = first_chunk<HAD>(tid) + k * nt;
+        const int c = first_chunk<RT, MAXV, MODE, HAD>(tid) + k * nt;
         const int64_t e = chunk_elem<SPLIT>(c);
         if constexpr ((HAD & HAD_MFMA) != 0)
         {
@@ -236,7 +254,7 @@ __device__ __forceinline__ void rms_load(const RmsArgs& a, int64_t row, int tid,
         #pragma unroll
         for (int k = 0; k < MAXV; ++k)
         {
-            const int c = first_chunk<HAD>(tid) + k * nt;
+            const int c = first_chunk<RT, MAXV, MODE, HAD>(tid) + k * nt;
             #pragma unroll
             for (int i = 0; i < kRowPre<HAD, MAXV>; ++i)
                 if (i < a.nh && a.hpre[i]) L.pv[k][i] = load8<TF16>(a.hpre[i], pre + (c < nc ? c * 8 : 0)).a;
@@ -430,8 +448,11 @@ __device__ __forceinline__ void rms_finish(const RmsArgs& a, int64_t row, int ti
     char* rrow = (char*)a.r + row * a.ldr * RT::bytes;
     char* yrow = (char*)a.y + row * a.ldy * YT::bytes;
     constexpr bool MF = (HAD & HAD_MFMA) != 0;
-    const int c0 = first_chunk<HAD>(tid);
+    const int c0 = first_chunk<RT, MAXV, MODE, HAD>(tid);
     const int lane = tid & 63;
+    constexpr bool kMove = kLaneOrder<RT, MAXV, MODE, HAD>;
+    // the first chunk that the transforms have in this lane
+    [[maybe_unused]] const int cm0 = kMove ? (tid & ~63) | mfma_chunk(lane) : c0;
     [[maybe_unused]] HadMfmaWords H{};
     if constexpr (MF)
     {
@@ -445,11 +466,17 @@ __device__ __forceinline__ void rms_finish(const RmsArgs& a, int64_t row, int ti
             #pragma unroll
             for (int k = 0; k < MAXV; ++k)
             {
-                const int c = c0 + k * nt;
+                const int c = cm0 + k * nt;
                 post[k] = c < nc ? a.hxpost : nullptr;
                 col[k] = (int64_t)c * 8;
+                if constexpr (kMove) L.xv[k] = mfma_permute(L.xv[k], lane);
             }
             output_rotations_mfma<MAXV>(H, L.xv, post, col, lane);
+            if constexpr (kMove)
+            {
+                #pragma unroll
+                for (int k = 0; k < MAXV; ++k) L.xv[k] = mfma_permute(L.xv[k], lane);
+            }
         }
     }
     // Pass 1: residual update and sum of squares.  The row is then cached in its narrowest exact
@@ -504,15 +531,23 @@ __device__ __forceinline__ void rms_finish(const RmsArgs& a, int64_t row, int ti
                 if constexpr (MAXV == 1) norm();
                 if constexpr (kDeferResidual<MODE, RT>)
                 {
-#ifdef EXL3R_TUNING
-                    if (a.r_cached) store8c<RT>(rrow, e, cache[k]);
+                    if constexpr (kMove) store8c<RT>(rrow, e, cache[k]);
                     else
+                    {
+#ifdef EXL3R_TUNING
+                        if (a.r_cached) store8c<RT>(rrow, e, cache[k]);
+                        else
 #endif
-                        store8<RT>(rrow, e, cache[k]);
+                            store8<RT>(rrow, e, cache[k]);
+                    }
                 }
                 if constexpr (MAXV != 1) norm();
                 if (a.y) store8<YT>(yrow, e, yv);
             }
+            TF16::Vec ym = yv;
+            if constexpr (kMove) ym = mfma_permute(yv, lane);
+            const bool mlive = cm0 + k * nt < nc;
+            const int64_t em = (int64_t)(cm0 + k * nt) * 8;
             // the consumers' transforms of this chunk (at most 4), their MFMAs issued together
             // (in pairs: four results at once would hold 32 more VGPRs and cost a wave per SIMD)
             #pragma unroll
@@ -525,12 +560,12 @@ __device__ __forceinline__ void rms_finish(const RmsArgs& a, int64_t row, int ti
                 for (int d = 0; d < 2; ++d)
                 {
                     const int i = i0 + d;
-                    v[d] = yv;
+                    v[d] = ym;
                     if (i < a.nh && a.hpre[i])   // (lanes past the row hold zeros)
                     {
                         u32x4 p;
                         if constexpr (kRowPre<HAD, MAXV> > 0) p = L.pv[k][i];
-                        else p = load8<TF16>(a.hpre[i], pre_row(a, row) + (live ? e : 0)).a;
+                        else p = load8<TF16>(a.hpre[i], pre_row(a, row) + (mlive ? em : 0)).a;
                         #pragma unroll
                         for (int q = 0; q < 4; ++q) v[d].a[q] = hmul2(v[d].a[q], (uint32_t)p[q]);
                     }
@@ -550,7 +585,9 @@ __device__ __forceinline__ void rms_finish(const RmsArgs& a, int64_t row, int ti
                     {
                         float f[8];
                         had128_mfma_finish(m[d], f, lane, a.hr);
-                        if (live) store8<TF16>((char*)a.hout[i] + row * a.ldh * 2, e, pack8<TF16>(f));
+                        TF16::Vec o = pack8<TF16>(f);
+                        if constexpr (kMove) o = mfma_permute(o, lane);
+                        if (live) store8<TF16>((char*)a.hout[i] + row * a.ldh * 2, e, o);
                     }
                 }
             }
@@ -972,17 +1009,19 @@ inline RmsShape rms_shape(int nc, int64_t rows, int mode, int had, bool wide = f
         return sh;
     }
 #endif
-    // Matrix-core Hadamard rows: one chunk per lane while 1024 lanes cover the row, the pre-scales held beside it
-    // (f16 x / f32 r, three outputs, rotated input, us for 1 / 2 / 4 chunks per lane: [4096, 5120] 69.0 / 73.4 /
-    // 76.1, [8192, 5120] 131.1 / 137.5 / 139.3, [4096, 2560] 35.6 / 38.0 / 39.4, [4096, 4096] 53.4 / 55.4 / 60.0).
-    // Two chunks per lane halve a row's waves, so where they let the launch run in one round of resident
-    // workgroups, with some room, and one chunk does not, they win ([1200, 5120] 20.1 against 25.8, [1100, 5120]
-    // 19.6 / 23.7; at 1500 of 1536 rows a round 30.9 / 29.6).
+    // Matrix-core Hadamard rows.  Two chunks per lane halve a row's waves, so where they let the launch run in one
+    // round of resident workgroups, with some room, and one chunk does not, they win (f32 residual [1200, 5120] 20.1
+    // against 25.8, [1100, 5120] 19.6 / 23.7; at 1500 of 1536 rows a round 30.9 / 29.6).  Otherwise f32 rows take one
+    // chunk per lane while 1024 lanes cover the row, the pre-scales held beside it, and 16-bit rows the rule of the
+    // other streaming norms (us for 1 / 2 chunks, three outputs, without and with rotated input: f32 residual
+    // [4096, 5120] 65.3 67.9 / 66.8 67.3, [2048, 8192] 51.9 53.4 / 53.8 55.3; f16 residual [4096, 5120] 49.0 55.3 / 47.3
+    // 50.6, [2048, 8192] 41.6 43.3 / 37.8 39.4; no residual [2000, 5120] 21.8 25.2 / 20.8 22.7, [2048, 8192] 33.0 34.9 /
+    // 29.7 32.5).
     if ((had & HAD_MFMA) && thr(1) <= 1024)
     {
         const int64_t round1 = (int64_t)(2048 / thr(1)) * device_cus(), round2 = (int64_t)(2048 / thr(2)) * device_cus();
         if (rows > round1 && rows <= round2 - round2 / 8) return { 2, thr(2), W_EARLY };
-        return { 1, thr(1), W_EARLY };
+        if (wide) return { 1, thr(1), W_EARLY };
     }
     if (rows > 1024 && mode == RMS_RES_IN && !had)
     {

@@ -12,7 +12,7 @@ import pytest
 import torch
 
 import exl3r.ffi as ffi
-from _gpu import NTHREADS, assert_bitwise, assert_close_ulp, assert_had_close, dev_normal, from_dev, to_dev
+from _gpu import NTHREADS, assert_bitwise, assert_close_ulp, assert_had_close, dev_normal, from_dev, graph_us, to_dev
 from oracle import oracle as orc
 from test_gpu_act_had import oracle_act, suh
 
@@ -263,6 +263,36 @@ def test_norm_had_launch_shapes(rows, dim):
     one round (769 to 1344 of 5120), rows past 1024 lanes (8320), and widths that end inside a 512-element span."""
     run_norm(rows, dim, F16, F32, n_out=4, with_y=False, rotate_x=True, seed=rows)
     run_norm(rows, dim, BF16, None, n_out=1, with_y=True, cb=1.0, seed=rows + 1)
+
+
+@pytest.mark.parametrize("rows,dim", [(769, 5120), (1100, 5248), (300, 16384), (1025, 8320)])
+@pytest.mark.parametrize("rt", [None, F16, F32])
+def test_norm_had_two_chunks_per_lane(rows, dim, rt):
+    """Two chunks per lane, by the round rule and in rows beyond 1024 chunks: owned in the transforms' placement, or
+    in lane order (f32 residual); the last lanes hold one chunk or none."""
+    run_norm(rows, dim, F16, rt, n_out=4, with_y=True, rotate_x=rt is not None, seed=rows)
+
+
+def norm_had_us(rows, dim, rt, rot):
+    x, w = dev_normal((rows, dim), 0, 1, F16, 1), dev_normal((dim,), 1, 0.1, F16, 2)
+    r = None if rt is None else dev_normal((rows, dim), 0, 4, rt, 3)
+    signs = torch.ones(dim, device="cuda", dtype=torch.float16)
+    outs = [torch.empty_like(x) for _ in range(3)]
+    return graph_us(lambda: ffi.rms_norm_had(x, w, outs, [signs] * 3, 1e-6, r=r, rotate_x=rot, x_post_scale=signs if rot else None))
+
+
+@pytest.mark.parametrize("rows,dim", [(4096, 5120), (2048, 8192)])
+def test_norm_had_16_bit_residual_in_proportion(rows, dim):
+    """A 16-bit residual moves 3/4 of an f32 one's bytes.  With its own chunks per lane it takes 0.74 of the time
+    (50.6 against 67.9 us at [4096, 5120]); with the f32 rows' one chunk per lane it took 0.81.  The rest is for the
+    clock."""
+    assert norm_had_us(rows, dim, F16, True) < 0.78 * norm_had_us(rows, dim, F32, True)
+
+
+def test_norm_had_two_chunk_f32_residual_in_proportion():
+    """An f32 residual moves 4/3 of a 16-bit one's bytes.  Rows of 16384 take 1.22 of the time in lane order with cached
+    residual stores (91.7 against 75.2 us), and took 1.41 in the transforms' placement."""
+    assert norm_had_us(2048, 16384, F32, False) < 1.32 * norm_had_us(2048, 16384, F16, False)
 
 
 @pytest.mark.parametrize("act,rot", [("silu", (True, True)), ("gelu", (False, False))])
