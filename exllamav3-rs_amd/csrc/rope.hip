@@ -1235,7 +1235,7 @@ void k_rope_nx(RopeArgs a, int nslice, int run, int early)
             const int64_t crow = cache_row_of();
             if (!isq && crow >= 0)
             {
-                char* cb = isv ? vcache : kcache;
+                char* cb = pick_qkv(false, isv, kcache, kcache, vcache);
                 const int64_t co = crow + (int64_t)hidx * HD + e0;
                 store8<IO>(cb, co, lo);
                 store8<IO>(cb, co + gap, hi);

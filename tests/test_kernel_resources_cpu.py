@@ -67,6 +67,8 @@ def matching(kernels, pattern):
 LIMITS = [
     # argmax, four chunks of aligned logits in flight
     (r"void k_argmax(_ws)?<\w+, true, 4, false>", 96, 0, 0),
+    # RoPE with the paged append: nothing in scratch
+    (r"void k_rope_nx<\w+, [12], [012], \d, false, 1, true, ", 128, 0, 0),
     # norms of eight chunks per lane: no row of outputs held beside the row itself
     (r"void k_rms_norm<(TF16|TBF16), \w+, (TF16|TBF16), 8, 1, 0, 2, false, double>", 98, 0, 0),
     (r"void k_rms_norm<(TF16|TBF16), TF32, TF32, 8, 1, 0, 2, false, double>", 128, 6, 28),
