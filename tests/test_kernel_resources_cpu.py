@@ -69,6 +69,9 @@ LIMITS = [
     (r"void k_argmax(_ws)?<\w+, true, 4, false>", 96, 0, 0),
     # RoPE with the paged append: nothing in scratch
     (r"void k_rope_nx<\w+, [12], [012], \d, false, 1, true, ", 128, 0, 0),
+    # bf16 GPT-J with f32 head norms from the {cos, sin} table, one and two passes per item
+    (r"void k_rope_nx<TBF16, 1, 2, 2, false, 1, false, 0, 8, false>", 80, 0, 0),
+    (r"void k_rope_nx<TBF16, 1, 2, 2, false, 2, false, 0, 8, false>", 96, 0, 0),
     # norms of eight chunks per lane: no row of outputs held beside the row itself
     (r"void k_rms_norm<(TF16|TBF16), \w+, (TF16|TBF16), 8, 1, 0, 2, false, double>", 98, 0, 0),
     (r"void k_rms_norm<(TF16|TBF16), TF32, TF32, 8, 1, 0, 2, false, double>", 128, 6, 28),
@@ -84,3 +87,9 @@ def test_resources(kernels, pattern, vgprs, spills, scratch):
             for n, k in matching(kernels, pattern).items()
             if k[".vgpr_count"] > vgprs or k[".vgpr_spill_count"] > spills or k[".private_segment_fixed_size"] > scratch}
     assert not over, over
+
+
+def test_scalar_registers_of_the_rotating_gptj_append(kernels):
+    """Its scalar registers are full: what does not fit is moved to and from vector lanes in the item loop."""
+    hits = matching(kernels, r"void k_rope_nx<TF16, 1, 0, 0, false, 1, true, 2, 8, false>")
+    assert all(k[".sgpr_spill_count"] <= 84 for k in hits.values()), {n: k[".sgpr_spill_count"] for n, k in hits.items()}
