@@ -1565,13 +1565,47 @@ static void launch_rope_nx_p(const RopeArgs& a, hipStream_t s)
 // half lines per access, and plain prefills of it stay with the wave-per-token kernel (f16 19.9 / 19.3 at 4096
 // tokens of 32 / 8 heads; at 500 tokens 4.3 / 5.1).
 static bool rope_tok_launch(const RopeArgs& a);
-static bool rope_nx_part_ok(const RopeArgs& a, int rope_mode)
+
+// Tokens from which a PART launch goes to the wave-per-token kernel instead: with a wave for every resident slot that
+// kernel walks a token's heads in whole lines, and the less there is to compute per head, or the more heads a token
+// has, the sooner it wins.  Times of this kernel over that one's at 1100 / 2048 / 3072 / 4096 / 8192 tokens (f16, 32 / 8
+// heads, 64 rotary, unless said):
+//   no head norm: heads of 64 .72 / .82 / .96 / 1.11 / 1.15 (bf16 1.24 at 4096), with the append .66 / .79 / .96 / 1.12 /
+//     1.15 (16 / 8 heads .62 / .67 / .77 / .80 / .95), of 128 with it .60 / .86 / 1.01 / 1.14 / 1.23 (64 / 8 heads 1.08
+//     at 3072), from the {cos, sin} table .69 / 1.07 / 1.16 / 1.22 / 1.23 (heads of 64 .82 / .93 / 1.16 / 1.23 / 1.17),
+//     q | g split .73 / 1.00 / 1.18 / 1.24 / 1.27 (heads of 64 .70 / .87 / .99 / 1.20 / 1.20)
+//   head norm: heads of 64 .63 / .80 / .79 / .92 / .91, with the append .58 / .73 / .91 / .98 / .91; q | g split of 128
+//     .58 / .78 / .94 / 1.05 / 1.06 (64 / 8 heads 1.12 at 4096, bf16 1.12 at 3072; 32 / 4 .82 at 4639); table .63 / .92 /
+//     .97 / 1.08 / 1.10
+//   heads of 256: full width at most 1.02 (bf16 head norm .73 / .90 / 1.00 / 1.08 / 1.02, q | g split 1.07 at 4096); 16 / 2
+//     heads, no norm .69 / .77 / .97 / 1.07 / 1.09, with the append .65 / .78 / .90 / .99 / 1.02, head norm .59 / .68 /
+//     .78 / .86 / .93
+// An angle table has no such kernel.
+static int64_t part_tokens(const RopeArgs& a, bool bf16)
+{
+    constexpr int64_t kNever = INT64_MAX;
+    const bool qout = a.oq_ts != a.q_ts || a.oq_hs != a.q_hs, norm = a.qw != nullptr, full = a.hd == 256 && a.R == 256;
+    const int work = (a.hq + a.hk) * a.hd;
+    if (a.table) return kNever;
+    if (norm && !a.cst)
+    {
+        if (qout && a.hd == 128) return bf16 && work >= 8192 ? 2560 : bf16 || work >= 5120 ? 3584 : kNever;
+        return bf16 && !a.kc && full ? 3584 : kNever;
+    }
+    if (full) return kNever;
+    if (a.cst) return norm ? 3072 : work >= 5120 ? 2048 : 2560;
+    if (a.kc) return a.hd == 256 ? kNever : work >= 8192 ? 3072 : work >= 2048 ? 3584 : 7168;
+    return !qout ? 3584 : work >= 4608 ? 2048 : 2560;
+}
+
+static bool rope_nx_part_ok(const RopeArgs& a, int rope_mode, bool bf16)
 {
     const bool plain = !a.cst && !a.table && !a.kc && a.oq_ts == a.q_ts && a.oq_hs == a.q_hs;
     if (a.hd == 128 && plain && rope_tok_launch(a)) return false;
     const Tuning& tu = tuning();
     if (tu.rope_nx < 0 || rope_mode != EXL3R_ROPE_NEOX || (a.hd != 64 && a.hd != 128 && a.hd != 256)) return false;
     if (tu.rope_tok != 0 && tu.rope_nx == 0) return false;   // a test forcing one of the other kernels
+    if (rope_tok_launch(a) && a.tokens >= part_tokens(a, bf16)) return false;
     if (a.kc && a.hv != a.hk) return false;
     if (a.tokens >= ((int64_t)1 << 31)) return false;
     return !a.cst || ((uintptr_t)a.cst & 15) == 0;
@@ -1807,7 +1841,7 @@ static void launch_rope_vec(const RopeArgs& a, int lph, hipStream_t s)
     }
     if constexpr (MODE == EXL3R_ROPE_NEOX)
     {
-        if (rope_nx_part_ok(a, MODE)) return launch_rope_nx_part<IO, NORM>(a, s);
+        if (rope_nx_part_ok(a, MODE, IO::code == DT_BF16)) return launch_rope_nx_part<IO, NORM>(a, s);
     }
     if (a.cst)
     {

@@ -137,20 +137,19 @@ def assert_head_close(got, exp, hd, what="", rel=2.0 ** -8, max_ulp=2, min_exact
 
 
 def graph_us(fn, n=10):
-    """Time of one call of fn in a HIP graph of n of them: the best of five replays."""
+    """Time of one call of fn in a HIP graph of n of them: the best of 30 replays, after as many to wake the clock."""
     fn()
     torch.cuda.synchronize()
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):
         for _ in range(n):
             fn()
-    best = float("inf")
-    for _ in range(5):
-        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    for _ in range(30):
         graph.replay()
-        a.record()
+    marks = [torch.cuda.Event(enable_timing=True) for _ in range(31)]
+    marks[0].record()
+    for m in marks[1:]:
         graph.replay()
-        b.record()
-        torch.cuda.synchronize()
-        best = min(best, a.elapsed_time(b) * 1e3 / n)
-    return best
+        m.record()
+    torch.cuda.synchronize()
+    return min(a.elapsed_time(b) for a, b in zip(marks, marks[1:])) * 1e3 / n

@@ -4,8 +4,12 @@ walks the items, in front of and behind the switch.  Sources: inv_freq, the tabl
 the paged append, each against the oracle at its own tests' tolerance."""
 import numpy as np
 import pytest
+import torch
 
 import exl3r
+import exl3r.ffi as ffi
+from _gpu import dev_normal, graph_us
+from exl3r import _lib
 from oracle import oracle as orc
 from test_gpu_rope import run as run_rope
 from test_gpu_rope_paged import layout, run as run_paged
@@ -59,3 +63,44 @@ def test_paged_append(hd, R, bsz, seq):
     sl[0] = 9 * 256 - seq + 1                          # the first sequence's last position is past its block table
     bt[-1, :] = pages + 1                              # the last sequence's pages are outside the pool
     run_paged(bsz, seq, 13, 3, hd, R, NEOX, BF16, 256, pages, 9, sl, bt, seed=R)
+
+
+@pytest.mark.parametrize("seq", [2047, 2048, 2560, 3583, 3584])
+def test_both_sides_of_the_token_rule(seq):
+    """Without a head norm, and for bf16 heads of 128 in the q | g split, launches of many tokens go to the kernel that
+    gives a wave whole tokens."""
+    run_rope(1, seq, 18, 3, 64, 64, NEOX, F16, norm=False, position=2, seed=seq)
+    run_qg(1, seq, 36, 4, 128, 64, NEOX, F16, position=5, seed=seq)
+    run_qg(1, seq, 18, 3, 128, 64, NEOX, BF16, nwt=BF16, cb=1.0, position=5, seed=seq)
+    pages, bt, sl = layout(1, seq, 256, 16, seq)
+    run_paged(1, seq, 40, 8, 64, 64, NEOX, F16, 256, pages, 16, sl, bt, norm=False, with_out_k=False, seed=seq)
+
+
+@pytest.mark.parametrize("hd,R,src", [(64, 64, "freq"), (64, 64, "table"), (64, 64, "append"), (128, 64, "table"),
+                                      (128, 64, "append"), (128, 64, "split")])
+@pytest.mark.parametrize("dt", [F16, BF16])
+@pytest.mark.parametrize("tokens", [1100, 4096])
+def test_the_token_rule_takes_the_faster_kernel(hd, R, src, dt, tokens):
+    """No head norm, 32 / 8 heads: at 4096 tokens the wave-per-token kernel is 1.1 to 1.4 times as fast as the 8-lane
+    layouts, at 1100 it is 0.6 to 0.9 times.  The launch's own choice, against that kernel forced (20% for the clock)."""
+    q, k = dev_normal((1, tokens, 32, hd), 0, 1, dt, 1), dev_normal((1, tokens, 8, hd), 0, 1, dt, 2)
+    inv = torch.rand(R // 2, device="cuda")
+    pages = torch.zeros((tokens // 256 + 2, 256, 8, hd), device="cuda", dtype=q.dtype)
+    kc, vc, table = pages, torch.zeros_like(pages), torch.arange(len(pages), dtype=torch.int32, device="cuda").view(1, -1)
+    lens = torch.zeros(1, dtype=torch.int32, device="cuda")
+    cs, qg = ffi.rope_cs_table(1, tokens, inv, 0), dev_normal((1, tokens, 32, 2 * hd), 0, 1, dt, 3)
+    out = torch.empty_like(q)
+    call = {
+        "freq": lambda: ffi.rope(q, q, k, k, inv, 0, None, None, None, 1e-6, 0.0, NEOX, 1.0),
+        "table": lambda: ffi.rope_cs(q, q, k, k, cs, None, None, 1e-6, 0.0, NEOX),
+        "append": lambda: ffi.rope_paged_kv(q, q, k, None, k, inv, 0, None, None, None, 1e-6, 0.0, NEOX, 1.0, kc, vc, table, lens),
+        "split": lambda: ffi.rope_qg(qg, out, k, k, inv, 0, None, None, None, 1e-6, 0.0, NEOX, 1.0),
+    }[src]
+    own = per_token = float("inf")
+    with _lib.tuned() as lib:
+        for _ in range(2):
+            lib.exl3r_tune_rope_tok(0, 0, 0)
+            own = min(own, graph_us(call))
+            lib.exl3r_tune_rope_tok(2, 0, 0)
+            per_token = min(per_token, graph_us(call))
+    assert own < 1.2 * per_token, (own, per_token)
