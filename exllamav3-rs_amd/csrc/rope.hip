@@ -16,13 +16,14 @@
 // Layout: a head of head_dim elements is held by LPH = head_dim / 8 lanes, 8 elements (16 bytes) per
 // lane, so a wave holds 64 / LPH heads (4 heads of 128).  The head sum is a DPP butterfly inside the
 // LPH-lane group; NeoX partners live R/16 lanes apart in the same group and are exchanged by DPP
-// (a rotation by 8 lanes for R = 128) or ds_bpermute, GPT-J partners sit in the same lane.  Heads of 64, 128
-// and 256 take k_rope_nx, which holds 16 elements per lane with every rotary pair in one lane; the others two
-// kernels: k_rope_tok (prefill NeoX) gives each wave whole tokens -- the token's sin/cos evaluated
-// once, one per lane, and its heads walked in software-pipelined batches; k_rope (decode, GPT-J)
-// flattens (token, head) items over workgroups that share the sin/cos of the tokens they span
-// through LDS.  exl3r_rope_cs_table evaluates the sin/cos of a forward pass once into a table
-// that exl3r_rope_cs's kernels (the same two) copy rows of, instead of evaluating them per layer.
+// (a rotation by 8 lanes for R = 128) or ds_bpermute, GPT-J partners sit in the same lane.  Heads of 128,
+// and NeoX heads of 64 and 256 and partial widths, take k_rope_nx, which holds 16 elements per lane with every
+// rotary pair in one lane (the latter up to some thousand tokens: part_tokens).  The rest goes to two kernels:
+// k_rope_tok (prefill NeoX) gives each wave whole tokens -- the token's sin/cos evaluated once, one per lane, and
+// its heads walked in software-pipelined batches; k_rope (decode, GPT-J) flattens (token, head) items over
+// workgroups that share the sin/cos of the tokens they span through LDS.  exl3r_rope_cs_table evaluates the
+// sin/cos of a forward pass once into a table that exl3r_rope_cs's kernels (the same three) copy rows of,
+// instead of evaluating them per layer.
 #include "abi.hpp"
 #include "common.cuh"
 #include "hadamard.cuh"
@@ -684,7 +685,8 @@ __global__ __launch_bounds__(256) void k_rope_tok(RopeArgs a)
     while (step(A, B) && step(B, A)) {}
 }
 
-// head_dim 128 at prefill sizes, NeoX with rotary_dim 128 (Qwen3, Llama) or GPT-J with any rotary_dim:
+// head_dim 128, at decode and prefill sizes, NeoX with rotary_dim 128 (Qwen3, Llama) or GPT-J with rotary_dim a
+// multiple of 4 (heads of 64 and 256 and partial NeoX widths in the PART layout, see the kernel):
 // 8 lanes per head, lane j of a head's group holding elements [8j, 8j + 8) and [64 + 8j, 64 + 8j + 8),
 // so every rotary pair sits in one lane -- NeoX (t, t + 64) across the two chunks, GPT-J (2t, 2t + 1)
 // inside a chunk -- with no partner exchange; the head sum is a 3-step DPP butterfly, and each 16-byte
@@ -1558,10 +1560,10 @@ static void launch_rope_nx_p(const RopeArgs& a, hipStream_t s)
 
 // Heads of 64 and 256, and partial rotary widths of 128 (NeoX): the same kernel with its PART layout (the
 // vector kernels' conditions hold: R % 16 == 0, 16-byte aligned heads).  MI355X, HIP graph, us, against the
-// wave-per-token kernel (flattened below 1024 tokens and for angle tables): q | g split, 16 / 2 heads of 256 with
-// 64 rotary, 4639 tokens bf16 19.6 / 20.9, f16 18.7 / 24.5, 300 tokens 4.1 / 4.5; 32 / 8 heads of 64 with the paged
-// append, 4096 tokens 13.4 / 17.4, 64 sequences of one token of 16 / 8 3.1 / 3.7; angle tables, 16 / 16 heads of 64,
-// 4096 tokens 9.0 / 13.2, 32 / 8 heads of 128 at full width 16.5 / 26.2.  A half-width rotation of 128 touches
+// wave-per-token kernel (flattened below 1024 tokens and for angle tables), with head norms: q | g split, 16 / 2 heads
+// of 256 with 64 rotary, 4639 tokens bf16 19.6 / 20.0, f16 18.5 / 24.5, 300 tokens 4.1 / 4.5; 32 / 8 heads of 64 with
+// the paged append, f16, 4096 tokens 13.3 / 14.0, 64 sequences of one token of 16 / 8 3.1 / 3.7; angle tables, 16 / 16
+// heads of 64, 4096 tokens 9.0 / 13.2, 32 / 8 heads of 128 at full width 16.5 / 26.2.  A half-width rotation of 128 touches
 // half lines per access, and plain prefills of it stay with the wave-per-token kernel (f16 19.9 / 19.3 at 4096
 // tokens of 32 / 8 heads; at 500 tokens 4.3 / 5.1).
 static bool rope_tok_launch(const RopeArgs& a);
@@ -1822,8 +1824,8 @@ static void launch_rope_tok(RopeArgs a, hipStream_t s)
     else go(std::integral_constant<int, 3>{});
 }
 
-// Prefill-sized NeoX launches (a wave per token still gives every CU several waves) take the
-// wave-per-token kernel.  GPT-J (C4 at rotary 64: 35.2 us flattened vs 37.5 us per token) and
+// What k_rope_nx does not take: prefill-sized NeoX launches (a wave per token still gives every CU several waves)
+// go to the wave-per-token kernel.  GPT-J (C4 at rotary 64: 35.2 us flattened vs 37.5 us per token) and
 // decode-sized launches take the flattened kernel: items per lane enough workgroups to fill 256 CUs
 // several times over, then up to four heads per lane so each wave keeps 4 KiB of loads in flight.
 template <class IO, int MODE, int NORM>
@@ -2001,7 +2003,8 @@ static bool rope_vec_ok(const RopeArgs& a, int rope_mode)
     return vec;
 }
 
-// Prefill-sized NeoX launches take the wave-per-token kernel (launch_rope_vec).
+// From here on a NeoX launch that k_rope_nx leaves takes the wave-per-token kernel, not the flattened one
+// (launch_rope_vec).
 static bool rope_tok_launch(const RopeArgs& a)
 {
     const Tuning& tu = tuning();
@@ -2171,9 +2174,9 @@ extern "C" int exl3r_had_r_128(const void* x, int dtype, int64_t ldx, void* out,
                                int64_t cols, const void* pre_scale, const void* post_scale, float scale, void* stream);
 
 // exl3r_rope with the q / k projections' output rotation first (Linear::forward's
-// had_r_128(y, y, None, svh), src/modules.rs:231, then RoPE::apply on y).  Prefill-sized NeoX launches
-// of f16 heads of 128 run it inside the wave-per-token kernel; anything else runs the rotations into
-// out_q / out_k and exl3r_rope in place there.
+// had_r_128(y, y, None, svh), src/modules.rs:231, then RoPE::apply on y).  f16 heads of 128 run it
+// inside k_rope_nx (rope_nx_ok: full-width NeoX or GPT-J, up to 192 heads), other prefill-sized NeoX launches of them
+// inside the wave-per-token kernel; anything else runs the rotations into out_q / out_k and exl3r_rope in place there.
 extern "C" int exl3r_rope_had(const void* q, void* out_q, int64_t q_tok_stride, int num_heads_q,
                               const void* k, void* out_k, int64_t k_tok_stride, int num_heads_k,
                               int dtype, int64_t bsz, int64_t seq_len, int head_dim,
@@ -2240,7 +2243,7 @@ extern "C" int exl3r_rope_had(const void* q, void* out_q, int64_t q_tok_stride, 
 
 // exl3r_rope_paged_kv preceded by the q / k / v projections' output rotation (Linear::forward's
 // had_r_128(y, y, None, svh), src/modules.rs:231, then RoPE::apply and paged_kv_cache_update,
-// src/modules.rs:669-704).  Prefill-sized NeoX launches of f16 heads of 128 run it inside the
+// src/modules.rs:669-704).  f16 heads of 128 run it inside k_rope_nx or, as exl3r_rope_had, the
 // wave-per-token kernel; anything else rotates q into out_q, k into out_k (in place when out_k is
 // null) and v in place, then runs exl3r_rope_paged_kv there.
 extern "C" int exl3r_rope_paged_kv_had(const void* q, void* out_q, int64_t q_tok_stride, int num_heads_q,

@@ -286,8 +286,8 @@ __device__ __forceinline__ typename IT::Vec load_chunk(const void* base, int64_t
 // is NaN or +inf where x is.  The slice's draw is then its logits' argmax, the first index where all are -inf.  (us in
 // a HIP graph, 16 / 64 rows of 151936 f32 logits, live 9.3 / 14.3, all but 50 columns of a row -inf 9.0 / 14.0, -1e9
 // 11.0 / 15.3, a NaN in every row 9.5 / 16.4; one by one with their noise 20.2 / 26.9, 20.2 / 25.1 and 21 / 25.3.)
-// 64 rows of 151936 f32 logits took 22.0 us with
-// every candidate exact, bound by VALU issue, and take 14.7 (three launches, ~13 us of host time from Python); 1024 rows 247 -> 122.5 us (5.1 TB/s).
+// 64 rows of 151936 f32 logits took 20.9 us in a HIP graph with every candidate exact, bound by VALU issue, and take
+// 14.2; 1024 rows 242 -> 122 us (5.1 TB/s).
 constexpr float kRankErr = 1e-5f;
 constexpr float kAbsorbs = 0x1.1p29f;
 

@@ -9,8 +9,8 @@ Exl3rError on a non-zero status (the reference's TORCH_CHECK raises).
 
 The wrappers of a forward pass hand their arguments to the native module first (_lib.fast, host/fast_ffi.cpp),
 which makes the call or declines it; what follows in the wrapper is the general form and has the errors.  A
-decode layer's four calls took 42.8 us through ctypes and take 14.9 through the native module, which is the
-GPU's own time for them."""
+decode layer's four calls took 42.8 us through ctypes and take 14.6 through the native module; the GPU needs
+11.8 us for them (one graph of the four), so such a layer is still bound by its host calls."""
 import ctypes
 import math
 
