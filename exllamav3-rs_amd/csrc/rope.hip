@@ -831,8 +831,12 @@ __device__ __forceinline__ double nx_head_sum(double v)
 // rotary width R of 16 m elements, R / 2 = 8 m apart.  Lane j < m of a head holds the chunks j and j + m,
 // whose elements pair up; lane j >= m holds the chunks m + j and L + j past the rotary width, which are
 // normed and pass through.  Every pair stays in one lane, as in the full-width layout, which is m = L.
+//
+// FORM: which of the two forms the instance holds, the one item per wave or the walk over the items at the kernel's
+// end.  NX_BOTH takes the form from the launch (early).
+enum { NX_BOTH = 0, NX_ONE = 1, NX_WALK = 2 };
 template <class IO, int MODE, int NORM, int SRC, bool QOUT, int P, bool APPEND = false, int HADR = HADR_NONE, int L = 8,
-          bool PART = false>
+          bool PART = false, int FORM = NX_BOTH>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kNxMinWaves<APPEND, HADR, SRC>)))
 void k_rope_nx(RopeArgs a, int nslice, int run, int early)
 {
@@ -1308,7 +1312,7 @@ void k_rope_nx(RopeArgs a, int nslice, int run, int early)
                      [&] { return APPEND ? t.crow : -1; }, std::false_type{});
     };
 
-    if constexpr (P == 1)
+    if constexpr (P == 1 && FORM != NX_WALK)
     {
     // Few items (a decode batch, a short prefill): every wave has one at most.  Such a launch is one chain of
     // latencies, so everything an item needs is loaded at once, the weights and post-scales straight into the
@@ -1317,7 +1321,7 @@ void k_rope_nx(RopeArgs a, int nslice, int run, int early)
     // of 64 / 8 heads, HIP graph, us before and after: 1 token 3.49 -> 2.86, 64 sequences 3.81 -> 3.55.  (Sending
     // the item's loads ahead of the LDS setup and then entering the loop below gained nothing: the loop's
     // registers are others, and moving a loaded value waits for it.)
-    if (early)
+    if (FORM == NX_ONE || early)
     {
         if (item0 >= items) return;
         Item A;
@@ -1506,6 +1510,7 @@ template <class IO, int MODE, int NORM, int SRC, bool QOUT, int P, bool APPEND =
 static void launch_rope_nx_p(const RopeArgs& a, hipStream_t s)
 {
     constexpr int HPP = 64 / L;
+    constexpr bool kFlat = SRC == SRC_CS && P == 1 && !APPEND && !HADR;   // see the grid below
     constexpr size_t kRows = SRC != SRC_CS ? 4 * (L == 16 ? 128 : 64) * sizeof(float2) : 0;   // {cos, sin} rows
     const int H = a.hq + a.hk + (APPEND ? a.hv : 0);
     const int nslice = ((H + HPP - 1) / HPP + P - 1) / P;
@@ -1519,8 +1524,9 @@ static void launch_rope_nx_p(const RopeArgs& a, hipStream_t s)
     // walking its items i, i + W, ...
     auto occupancy = [](size_t bytes) {
         int nb = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_rope_nx<IO, MODE, NORM, SRC, QOUT, P, APPEND, HADR, L, PART>,
-                                                         256, bytes) != hipSuccess || nb < 1)
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
+                &nb, k_rope_nx<IO, MODE, NORM, SRC, QOUT, P, APPEND, HADR, L, PART, kFlat ? NX_WALK : NX_BOTH>, 256,
+                bytes) != hipSuccess || nb < 1)
             nb = 4;
         return nb;
     };
@@ -1528,7 +1534,8 @@ static void launch_rope_nx_p(const RopeArgs& a, hipStream_t s)
     const int resident = lds <= kLdsCommon ? resident_common : occupancy(lds);
     const int wpc = tuning().rope_wgs_per_cu;
     int64_t blocks = (int64_t)(wpc > 0 ? wpc : resident) * device_cus();
-    const bool few = items <= blocks * 4;      // a wave per item at most
+    const int64_t resident_waves = blocks * 4;
+    const bool few = items <= resident_waves;  // a wave per item at most
     // Items a wave takes in a row, its token's angles evaluated once within them, where every wave gets
     // whole runs (prefill sizes).  MI355X, same process, us at runs of 1 / 2 / 3: C4 NeoX 33.2 / 32.1 /
     // 33.3; q / k rotations + RoPE at C4 46.8 / 45.5 / 42.7; q / k / v rotations + RoPE + paged append at
@@ -1547,15 +1554,31 @@ static void launch_rope_nx_p(const RopeArgs& a, hipStream_t s)
     // Plain passes reading the {cos, sin} table carry nothing from one item to the next: a wave per
     // run over the whole grid, dispatched as workgroups retire, beats the resident grid (C4, same
     // process: 30.8 vs 32.1 us; the evaluated and the GPT-J passes lose with it, 37.5 / 35.7 us).
-    constexpr bool kFlat = SRC == SRC_CS && P == 1 && !APPEND && !HADR;
     if (kFlat && wpc == 0) blocks = (runs + 3) / 4;
     if (blocks > (runs + 3) / 4) blocks = (runs + 3) / 4;
     if (blocks > kMaxGridX) blocks = kMaxGridX;
     RopeArgs b = a;
     udiv_magic_init((uint64_t)nslice, b.ns_m, b.ns_l);
     const int early = P == 1 && few && run == 1;
-    launch(k_rope_nx<IO, MODE, NORM, SRC, QOUT, P, APPEND, HADR, L, PART>, (unsigned)blocks, 256, lds, s, b, nslice, run,
-           early);
+    if constexpr (kFlat)
+    {
+        // Flat grids have an item per wave, so the one-item form takes them at every size: no LDS setup, no barrier, and
+        // registers for eight waves per SIMD (C4 28.7 us against 30.7 - 32.3 from the walking form).  With f32 head
+        // norms its weights are 64 bytes per lane to load in front of each item, which pays up to two rounds of
+        // resident waves (bf16, one item / walking, us: 64 / 8 heads, 700 tokens 6.1 / 7.1, 1100 10.2 / 10.4, 2048
+        // 16.9 / 15.7, 16384 110 / 102).  Each form has an instance of its own: in one kernel with the other the walking
+        // form took 3 to 6% longer with head norms (f16 64 / 8 heads, 4639 tokens 32.3 / 31.1, bf16 32.2 / 31.4).
+        const bool one = run == 1 && blocks * 4 >= items && (NORM != NORM_F32 || items <= 2 * resident_waves);
+        if (one)
+            launch(k_rope_nx<IO, MODE, NORM, SRC, QOUT, P, APPEND, HADR, L, PART, NX_ONE>, (unsigned)blocks, 256, lds, s, b,
+                   nslice, run, 1);
+        else
+            launch(k_rope_nx<IO, MODE, NORM, SRC, QOUT, P, APPEND, HADR, L, PART, NX_WALK>, (unsigned)blocks, 256, lds, s,
+                   b, nslice, run, 0);
+    }
+    else
+        launch(k_rope_nx<IO, MODE, NORM, SRC, QOUT, P, APPEND, HADR, L, PART>, (unsigned)blocks, 256, lds, s, b, nslice,
+               run, early);
 }
 
 // Heads of 64 and 256, and partial rotary widths of 128 (NeoX): the same kernel with its PART layout (the

@@ -104,3 +104,45 @@ def test_the_token_rule_takes_the_faster_kernel(hd, R, src, dt, tokens):
             lib.exl3r_tune_rope_tok(2, 0, 0)
             per_token = min(per_token, graph_us(call))
     assert own < 1.2 * per_token, (own, per_token)
+
+
+@pytest.mark.parametrize("hq,hk", [(18, 3), (64, 8)])
+@pytest.mark.parametrize("dt,nwt", [(F16, F16), (F16, F32), (BF16, BF16), (F16, None), (BF16, None)])
+@pytest.mark.parametrize("tokens", [1, 7, 500, 1400, 1600, 4100])
+def test_forms_from_the_table(hq, hk, dt, nwt, tokens):
+    """RoPE from the {cos, sin} table, one item per wave or a walk over the items (f32 weights in the kernel beyond two
+    rounds of resident waves: 1365 tokens of 64 / 8 heads), against the evaluated angles, which give the same bits."""
+    q, k = dev_normal((1, tokens, hq, 128), 0, 1, dt, tokens), dev_normal((1, tokens, hk, 128), 0, 1, dt, hq)
+    qn = kn = None
+    if nwt is not None:
+        qn, kn = dev_normal((128,), 1, 0.1, nwt, 3), dev_normal((128,), 1, 0.1, nwt, 4)
+    inv = torch.rand(64, device="cuda")
+    for mode in (NEOX, exl3r.ROPE_GPTJ):
+        want = [torch.empty_like(q), torch.empty_like(k)]
+        got = [torch.empty_like(q), torch.empty_like(k)]
+        ffi.rope(q, want[0], k, want[1], inv, 3, None, qn, kn, 1e-6, 0.0, mode, 1.0)
+        cs = ffi.rope_cs_table(1, tokens, inv, 3)
+        ffi.rope_cs(q, got[0], k, got[1], cs, qn, kn, 1e-6, 0.0, mode)
+        for a, b in zip(got, want):
+            assert torch.equal(a.view(torch.int16), b.view(torch.int16)), mode
+
+
+def test_the_table_is_faster_than_the_angles():
+    """4639 tokens of 64 / 8 f16 heads with norms: 28.7 us from the table against 32.5 evaluated (32.3 when both forms
+    shared an instance and flat grids walked).  Four buffers in turn, more than the caches hold."""
+    bufs = [(dev_normal((1, 4639, 64, 128), 0, 1, F16, i), dev_normal((1, 4639, 8, 128), 0, 1, F16, 9 + i)) for i in range(4)]
+    n, inv = dev_normal((128,), 1, 0.1, F16, 3), torch.rand(64, device="cuda")
+    cs = ffi.rope_cs_table(1, 4639, inv, 0)
+
+    def table():
+        for q, k in bufs:
+            ffi.rope_cs(q, q, k, k, cs, n, n, 1e-6, 0.0, NEOX)
+
+    def angles():
+        for q, k in bufs:
+            ffi.rope(q, q, k, k, inv, 0, None, n, n, 1e-6, 0.0, NEOX, 1.0)
+
+    read = evaluated = float("inf")
+    for _ in range(3):
+        read, evaluated = min(read, graph_us(table, 5)), min(evaluated, graph_us(angles, 5))
+    assert read < 0.95 * evaluated, (read, evaluated)
