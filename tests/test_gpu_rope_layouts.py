@@ -146,3 +146,22 @@ def test_the_table_is_faster_than_the_angles():
     for _ in range(3):
         read, evaluated = min(read, graph_us(table, 5)), min(evaluated, graph_us(angles, 5))
     assert read < 0.95 * evaluated, (read, evaluated)
+
+
+def test_gptj_from_the_table_is_as_fast_in_bf16():
+    """4639 tokens of 16 / 8 heads without norms: 10.8 us in f16 and in bf16, whose instance took 11.6."""
+    inv = torch.rand(32, device="cuda")
+    cs = ffi.rope_cs_table(1, 4639, inv, 0)
+
+    def over(dt):
+        bufs = [(dev_normal((1, 4639, 16, 128), 0, 1, dt, i), dev_normal((1, 4639, 8, 128), 0, 1, dt, 9 + i)) for i in range(8)]
+
+        def call():
+            for q, k in bufs:
+                ffi.rope_cs(q, q, k, k, cs, None, None, 1e-6, 0.0, exl3r.ROPE_GPTJ)
+        return call
+
+    half, brain = over(F16), over(BF16)
+    times = [(graph_us(half, 5), graph_us(brain, 5)) for _ in range(3)]
+    half_us, brain_us = (min(t) for t in zip(*times))
+    assert brain_us < 1.04 * half_us, (half_us, brain_us)
